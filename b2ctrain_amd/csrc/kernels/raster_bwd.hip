@@ -91,15 +91,15 @@ __global__ void __launch_bounds__(64) raster_bwd_fp32_kernel(b2c_raster_bwd_args
   __shared__ float4 s_geo[64], s_shape[64], s_rgb[64];  // proj0, proj1, proj2 of the batch's splats
   __shared__ float2 s_f3[FEAT ? 64 : 1];                  // proj3 (feature y, z)
   __shared__ uint32_t s_id[64];
-  const int n_tiles = a.tiles_x * a.tiles_y;
-  const int tile = xcd_tile(blockIdx.x, n_tiles);
-  if (tile >= n_tiles) return;
+  const TileAt here = xcd_tile(blockIdx.x, a.tiles_x, a.tiles_y);
+  const int tile = here.tile;
+  if (tile < 0) return;
   const uint2 range = reinterpret_cast<const uint2*>(a.tile_ranges)[tile];
   if (range.y <= range.x) return;
   const int lane = threadIdx.x;
-  const int px = (tile % a.tiles_x) * RT_W + (lane & 7), py = (tile / a.tiles_x) * RT_W + (lane >> 3);
+  const int px = here.tx * RT_W + (lane & 7), py = here.ty * RT_W + (lane >> 3);
   const PixelState ps = load_pixel<FEAT, HOLLOW>(a, px, py, range.x, a.last_idx);
-  const float tcx = (tile % a.tiles_x) * RT_W + RT_W * 0.5f, tcy = (tile / a.tiles_x) * RT_W + RT_W * 0.5f;
+  const float tcx = here.tx * RT_W + RT_W * 0.5f, tcy = here.ty * RT_W + RT_W * 0.5f;
   const PixelPoly pp = pixel_poly(ps.pcx - tcx, ps.pcy - tcy);
   const float Wf = (float)a.W, Hf = (float)a.H;
   float T = ps.T;
@@ -276,9 +276,9 @@ __global__ void __launch_bounds__(64) raster_bwd_mfma_kernel(b2c_raster_bwd_args
   // the refine products, already the fp16 operand of their MFMA (truncated as the conversion of fp32 rows
   // would be)
   __shared__ __attribute__((aligned(16))) _Float16 sR[G][SROW_H];
-  const int n_tiles = a.tiles_x * a.tiles_y;
-  const int tile = xcd_tile(blockIdx.x, n_tiles);
-  if (tile >= n_tiles) return;
+  const TileAt here = xcd_tile(blockIdx.x, a.tiles_x, a.tiles_y);
+  const int tile = here.tile;
+  if (tile < 0) return;
   // with the forward's compacted lists: the entries some pixel composited, the pixels' ends in them
   const bool compact = a.cvals != nullptr;  // uniform
   uint2 range = reinterpret_cast<const uint2*>(a.tile_ranges)[tile];
@@ -289,7 +289,7 @@ __global__ void __launch_bounds__(64) raster_bwd_mfma_kernel(b2c_raster_bwd_args
   // pairs past the shrunk end (or left out of the compacted list) never composited: they get no row, and the
   // reduce does not read theirs
   if (range.y <= range.x) return;
-  const int tx = tile % a.tiles_x, ty = tile / a.tiles_x;
+  const int tx = here.tx, ty = here.ty;
   const int lx = lane & 7, ly = lane >> 3;
   const int px = tx * RT_W + lx, py = ty * RT_W + ly;
   const float u = lx + 0.5f - RT_W * 0.5f, v = ly + 0.5f - RT_W * 0.5f;  // offset from the tile centre
@@ -801,7 +801,7 @@ using namespace b2c::dev;
 extern "C" int b2c_hip_raster_bwd(const b2c_raster_bwd_args* a, hipStream_t stream) {
   const int n_tiles = a->tiles_x * a->tiles_y;
   if (n_tiles <= 0) return 0;
-  const dim3 grid(NUM_XCD * xcd_tiles_per(n_tiles)), block(64);
+  const dim3 grid(xcd_grid(a->tiles_x, a->tiles_y)), block(64);
   const bool feat = a->feat != 0, hollow = a->hollow_z != nullptr && a->hollow_lam != 0.f;
   if (feat && !a->v_feat) return (int)hipErrorInvalidValue;
   if (a->defer_vis && (a->mode != 1 || feat || !a->v_splat_zero)) return (int)hipErrorInvalidValue;

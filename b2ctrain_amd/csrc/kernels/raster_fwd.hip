@@ -35,12 +35,12 @@ __global__ void __launch_bounds__(64) raster_fwd_kernel(b2c_raster_fwd_args a) {
   __shared__ float4 s_ext[EXT ? 65 : 1];  // (feature xyz, camera depth)
   __shared__ uint32_t s_list[4][66];  // per quadrant: LDS byte offsets of its splats, in depth order
   __shared__ uint32_t s_flag[COMPACT ? 65 : 1];  // COMPACT: splat j of the batch was composited (64: the null splat)
-  const int n_tiles = a.tiles_x * a.tiles_y;
-  const int tile = xcd_tile(blockIdx.x, n_tiles);
-  if (tile >= n_tiles) return;
+  const TileAt here = xcd_tile(blockIdx.x, a.tiles_x, a.tiles_y);
+  const int tile = here.tile;
+  if (tile < 0) return;
   const int lane = threadIdx.x;
   const int q = lane >> 4, p = lane & 15;
-  const int tx = tile % a.tiles_x, ty = tile / a.tiles_x;
+  const int tx = here.tx, ty = here.ty;
   const int px = tx * RT_W + (q & 1) * 4 + (p & 3), py = ty * RT_W + (q >> 1) * 4 + (p >> 2);
   const float x0 = tx * RT_W + 0.5f, y0 = ty * RT_W + 0.5f;  // the tile's first pixel centre
   const bool inside = px < a.W && py < a.H;
@@ -219,7 +219,7 @@ extern "C" int b2c_hip_raster_fwd(const b2c_raster_fwd_args* a, hipStream_t stre
   const int n_tiles = a->tiles_x * a->tiles_y;
   if (n_tiles <= 0) return 0;
   if (!a->raster_rec || (a->hollow_z && !a->hollow_pen)) return (int)hipErrorInvalidValue;
-  const dim3 grid(NUM_XCD * xcd_tiles_per(n_tiles)), block(64);
+  const dim3 grid(xcd_grid(a->tiles_x, a->tiles_y)), block(64);
   const bool hollow = a->hollow_z != nullptr;
   const bool compact = a->bwd_info && a->cvals != nullptr;
   if (compact && (!a->cslots || !a->slot_sorted || !a->clast || !a->cend)) return (int)hipErrorInvalidValue;

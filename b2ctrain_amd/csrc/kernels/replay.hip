@@ -39,19 +39,19 @@ __global__ void __launch_bounds__(64) evidence_kernel(b2c_evidence_args a) {
   __shared__ __attribute__((aligned(16))) float s_kc[LABELS ? MAXC : 1][64];  // k of the tile's c-th class's pixels, else 0
   __shared__ uint32_t s_lab[64];                 // class of the pixels beyond the first MAXC classes
   __shared__ uint32_t s_slot[64];
-  const int n_tiles = a.tiles_x * a.tiles_y;
-  const int tile = xcd_tile(blockIdx.x, n_tiles);
-  if (tile >= n_tiles) return;
+  const TileAt here = xcd_tile(blockIdx.x, a.tiles_x, a.tiles_y);
+  const int tile = here.tile;
+  if (tile < 0) return;
   const uint2 range = reinterpret_cast<const uint2*>(a.tile_ranges)[tile];
   const int lane = threadIdx.x;
   float4* rows = reinterpret_cast<float4*>(a.rows);
   // entries past the shrunk end composited nowhere: they get no row (the sum reads a row without this
   // pass's tag as zero)
   if (range.y <= range.x) return;
-  const int px = (tile % a.tiles_x) * RT_W + (lane & 7), py = (tile / a.tiles_x) * RT_W + (lane >> 3);
+  const int px = here.tx * RT_W + (lane & 7), py = here.ty * RT_W + (lane >> 3);
   const bool inside = px < a.W && py < a.H;
   const float pcx = px + 0.5f, pcy = py + 0.5f;
-  const float tcx = (tile % a.tiles_x) * RT_W + RT_W * 0.5f, tcy = (tile / a.tiles_x) * RT_W + RT_W * 0.5f;
+  const float tcx = here.tx * RT_W + RT_W * 0.5f, tcy = here.ty * RT_W + RT_W * 0.5f;
   const PixelPoly pp = pixel_poly(pcx - tcx, pcy - tcy);
   float m = 0.f, mres = 0.f, k = 0.f;
   uint32_t last = range.x, lab = LABEL_NONE;
@@ -252,13 +252,13 @@ __global__ void __launch_bounds__(64) probe_kernel(b2c_probe_args a) {
   __shared__ float4 s_g0[65], s_g1[65];
   __shared__ float s_z[65];  // camera depth
   __shared__ uint32_t s_list[4][66];  // per quadrant: LDS byte offsets of its splats, in depth order
-  const int n_tiles = a.tiles_x * a.tiles_y;
-  const int tile = xcd_tile(blockIdx.x, n_tiles);
-  if (tile >= n_tiles) return;
+  const TileAt here = xcd_tile(blockIdx.x, a.tiles_x, a.tiles_y);
+  const int tile = here.tile;
+  if (tile < 0) return;
   const uint2 range = reinterpret_cast<const uint2*>(a.tile_ranges)[tile];
   const int lane = threadIdx.x;
   const int q = lane >> 4, p = lane & 15;
-  const int tx = tile % a.tiles_x, ty = tile / a.tiles_x;
+  const int tx = here.tx, ty = here.ty;
   const int px = tx * RT_W + (q & 1) * 4 + (p & 3), py = ty * RT_W + (q >> 1) * 4 + (p >> 2);
   const float x0 = tx * RT_W + 0.5f, y0 = ty * RT_W + 0.5f;  // the tile's first pixel centre
   const bool inside = px < a.W && py < a.H;
@@ -357,7 +357,7 @@ extern "C" int b2c_hip_evidence_view(const b2c_evidence_args* a, hipStream_t str
   const bool feat = a->normals && a->normal_weight > 0.f;
   const bool labels = a->labels && a->label_acc;
   if (feat && !a->out_feat) return (int)hipErrorInvalidValue;
-  const dim3 grid(NUM_XCD * xcd_tiles_per(n_tiles)), block(64);
+  const dim3 grid(xcd_grid(a->tiles_x, a->tiles_y)), block(64);
   if (feat) {
     if (labels) evidence_kernel<true, true><<<grid, block, 0, stream>>>(*a);
     else evidence_kernel<true, false><<<grid, block, 0, stream>>>(*a);
@@ -383,6 +383,6 @@ extern "C" int b2c_hip_probe_depth(const b2c_probe_args* a, hipStream_t stream) 
   const int n_tiles = a->tiles_x * a->tiles_y;
   if (n_tiles <= 0) return 0;
   if (!a->raster_rec || !a->out) return (int)hipErrorInvalidValue;
-  probe_kernel<<<dim3(NUM_XCD * xcd_tiles_per(n_tiles)), dim3(64), 0, stream>>>(*a);
+  probe_kernel<<<dim3(xcd_grid(a->tiles_x, a->tiles_y)), dim3(64), 0, stream>>>(*a);
   return (int)hipGetLastError();
 }
