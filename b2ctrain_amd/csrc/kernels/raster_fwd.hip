@@ -18,15 +18,37 @@ namespace {
 // reaches no pixel of a quadrant would contribute alpha = 0 there, so the result equals the plain sweep.
 // The loop is branch-free: a lane that has terminated, has run out of its list, or whose fragment fails
 // the cutoff contributes alpha = 0, which leaves T, the colour and the last index unchanged. Per splat the
-// LDS holds (D, E, F, c00/2), (c01, log2 opacity, power, c11/2) and the colour clamped at 0, staged from
+// LDS holds (D, E, F, c00/2), (c01, log2 opacity, -, c11/2) and (colour clamped at 0, power), staged from
 // the projection's 64-byte per-splat record (one cache line per gather): sigma is the tile-centred
 // quadratic of raster_common.h (sigma_coefs once per splat and tile, poly_sigma per fragment).
+//
+// The loop is bound by the LDS about as much as by the VALU: a CU's LDS was busy 68% of the kernel. A wave's
+// 16-byte read takes it 4.1 cycles and an 8-byte one 2.1, but a 12-byte read 8.2, which is what three used
+// lanes of a float4 compile to. So the third quarter carries the power in its fourth lane and the second
+// quarter's gap lies inside (two 8-byte reads): 184 -> 176 us on 1M splats at 1080p, 504 -> 460 us at 4K with large
+// splats, 387 -> 354 us on a dense slab of 3M.
 
 // COMPACT: the tile's compacted list for the MFMA backward (the entries some pixel composited). Each lane
 // marks the steps of its quadrant's list where it composited (one bit per step pair, even and odd steps
 // apart); after the batch the marks are OR-ed over the quadrant's 16 lanes, each lane flags in LDS the
 // splats at four of its quadrant's list positions that the quadrant composited, and splat j of the batch
 // is kept when some quadrant flagged it.
+struct FwdFrag {
+  float sigma, alpha;  // alpha capped, whatever sigma
+  float4 col;          // (colour, power)
+};
+
+__device__ __forceinline__ FwdFrag fwd_frag(const char* lds_g0, const char* lds_g1, const char* lds_col, uint32_t off,
+                                            const PixelPoly& pp) {
+  const float4 g0 = *reinterpret_cast<const float4*>(lds_g0 + off);
+  const float4 g1 = *reinterpret_cast<const float4*>(lds_g1 + off);
+  FwdFrag f;
+  f.col = *reinterpret_cast<const float4*>(lds_col + off);
+  f.sigma = poly_sigma(g0.w, g1.x, g1.w, g0.x, g0.y, g0.z, pp);
+  f.alpha = fminf(ALPHA_MAX, fragment_alpha(f.sigma, g1.y));
+  return f;
+}
+
 template <bool FEAT, bool HOLLOW, bool COMPACT>
 __global__ void __launch_bounds__(64) raster_fwd_kernel(b2c_raster_fwd_args a) {
   constexpr bool EXT = FEAT || HOLLOW;
@@ -81,8 +103,8 @@ __global__ void __launch_bounds__(64) raster_fwd_kernel(b2c_raster_fwd_args a) {
       const float4 r0 = rec[0], r1 = rec[1], r2 = rec[2];
       const float3 def = sigma_coefs(r0.x, r0.y, r0.z, r0.w, r1.x, tcx, tcy);
       s_g0[lane] = make_float4(def.x, def.y, def.z, r0.z);
-      s_g1[lane] = make_float4(r0.w, r2.w, r1.z, r1.x);
-      s_col[lane] = r2;
+      s_g1[lane] = make_float4(r0.w, r2.w, 0.f, r1.x);
+      s_col[lane] = make_float4(r2.x, r2.y, r2.z, r1.z);
       if constexpr (EXT) s_ext[lane] = rec[3];
       qmask = quadrant_mask(r0.x, r0.y, r0.z, r0.w, r1.x, r1.z, x0, y0);
     }
@@ -109,29 +131,25 @@ __global__ void __launch_bounds__(64) raster_fwd_kernel(b2c_raster_fwd_args a) {
     // n_pairs step pairs bit b stands for pair n_pairs - 1 - b. They give the lane's last composited entry
     // (and, COMPACT, the kept entries) without a select per step.
     uint32_t marks_even = 0, marks_odd = 0;
-    // One step: sigma <= power (a NaN sigma fails), bitwise & so the compiler does not branch on the
-    // compares; the exp is kept out of an exec-masked branch (a lane whose fragment fails has its alpha
-    // discarded by the select); only a valid fragment can stop a lane. The transmittance after a fragment is
-    // fma(-alpha, T, T): T (1 - alpha) rounded once (the depth probe's walk does the same). A fragment is
-    // composited (vis > 0) exactly when it is valid and does not stop the lane: a valid alpha is at least
-    // 1/255 and a live lane's T is above the cutoff.
-#define B2C_COMPOSITE(off, next, marks)                                                                \
+    // A step in two halves. fwd_frag needs no transmittance; both steps of a pair run it first, so their
+    // exponentials issue back to back (an exponential between other operations costs 13 cycles, the second of
+    // two 8). The exps are kept out of an exec-masked branch (a lane whose fragment fails has its alpha
+    // discarded by the select). Then, per step: sigma <= power (a NaN sigma fails), bitwise & so the compiler
+    // does not branch on the compares; only a valid fragment can stop a lane. The transmittance after a
+    // fragment is fma(-alpha, T, T): T (1 - alpha) rounded once (the depth probe's walk does the same). A
+    // fragment is composited (vis > 0) exactly when it is valid and does not stop the lane: a valid alpha is
+    // at least 1/255 and a live lane's T is above the cutoff.
+#define B2C_COMPOSITE(f, off, next, marks)                                                             \
   do {                                                                                                 \
-    const float4 g0 = *reinterpret_cast<const float4*>(lds_g0 + (off));                                \
-    const float4 g1 = *reinterpret_cast<const float4*>(lds_g1 + (off));                                \
-    const float4 col = *reinterpret_cast<const float4*>(lds_col + (off));                              \
-    const float sigma = poly_sigma(g0.w, g1.x, g1.w, g0.x, g0.y, g0.z, pp);                            \
-    const bool valid = live & (sigma <= g1.z);                                                         \
-    float a_cl = fminf(ALPHA_MAX, fragment_alpha(sigma, g1.y));                                        \
-    asm volatile("" : "+v"(a_cl));                                                                     \
-    const float alpha = valid ? a_cl : 0.f;                                                            \
-    const float next_T = __builtin_fmaf(-alpha, T, T);                                                      \
+    const bool valid = live & ((f).sigma <= (f).col.w);                                                \
+    const float alpha = valid ? (f).alpha : 0.f;                                                       \
+    const float next_T = __builtin_fmaf(-alpha, T, T);                                                 \
     const bool stop = next_T <= T_CUTOFF;                                                              \
     live = live & !stop;                                                                               \
     const float vis = stop ? 0.f : alpha * T;                                                          \
-    r += col.x * vis;                                                                                  \
-    g += col.y * vis;                                                                                  \
-    b += col.z * vis;                                                                                  \
+    r += (f).col.x * vis;                                                                              \
+    g += (f).col.y * vis;                                                                              \
+    b += (f).col.z * vis;                                                                              \
     if constexpr (EXT) {                                                                               \
       const float4 ext = *reinterpret_cast<const float4*>(lds_ext + (off));                            \
       if constexpr (FEAT) {                                                                            \
@@ -146,8 +164,11 @@ __global__ void __launch_bounds__(64) raster_fwd_kernel(b2c_raster_fwd_args a) {
     (off) = my_list[next];                                                                             \
   } while (0)
     for (uint32_t i = 0; i < n_iter; i += 2) {
-      B2C_COMPOSITE(off0, i + 2, marks_even);
-      B2C_COMPOSITE(off1, i + 3, marks_odd);
+      FwdFrag even = fwd_frag(lds_g0, lds_g1, lds_col, off0, pp);
+      FwdFrag odd = fwd_frag(lds_g0, lds_g1, lds_col, off1, pp);
+      asm volatile("" : "+v"(even.alpha), "+v"(odd.alpha));
+      B2C_COMPOSITE(even, off0, i + 2, marks_even);
+      B2C_COMPOSITE(odd, off1, i + 3, marks_odd);
     }
 #undef B2C_COMPOSITE
     const int n_pairs = (int)(n_iter + 1u) >> 1;
