@@ -2,6 +2,8 @@
 // host loop over views and the downloads; the replays are kernels/replay.hip.
 #include "evidence.h"
 
+#include <algorithm>
+
 namespace b2c {
 
 namespace {
@@ -9,6 +11,10 @@ namespace {
 DevBuf<float> g_evidence;  // [n][B2C_EVIDENCE_STRIDE]
 DevBuf<float> g_view_acc;  // [n][3] the current view's (w_in, err, w_all)
 DevBuf<float> g_labels;    // [n][B2C_LABEL_BINS]
+// The downloads' rows, formed on the device from the accumulators (sized with them; every download of one
+// pass writes the same values).
+DevBuf<float> g_evidence_rows;  // [n][7]
+DevBuf<float> g_label_rows;     // [n][2]
 bool g_labels_valid = false;
 }  // namespace
 
@@ -18,11 +24,13 @@ void compute_evidence(RenderCtx& ctx, const Model& m, const std::vector<ViewGPU>
   const size_t n = (size_t)(m.n > 0 ? m.n : 1);
   g_evidence.reserve(n * B2C_EVIDENCE_STRIDE);
   g_evidence.zero(stream);
+  g_evidence_rows.reserve(n * 7);
   g_view_acc.reserve(n * 3);
   g_labels_valid = cfg.export_labels;
   if (g_labels_valid) {
     g_labels.reserve(n * B2C_LABEL_BINS);
     g_labels.zero(stream);
+    g_label_rows.reserve(n * 2);
   }
   const bool use_normals = cfg.evidence_normal_weight > 0.f;
   for (size_t v = 0; v < views.size(); v++) {
@@ -75,46 +83,37 @@ const float* evidence_device(int* stride) {
   return g_evidence.ptr;
 }
 
-std::vector<float> download_evidence(const Model& m, hipStream_t stream) {
+void download_evidence(const Model& m, float* out, hipStream_t stream) {
   const size_t n = (size_t)m.n;
-  std::vector<float> out(n * 7, 0.f);
-  if (g_evidence.count < n * B2C_EVIDENCE_STRIDE || n == 0) return out;
-  const std::vector<float> acc = g_evidence.download(n * B2C_EVIDENCE_STRIDE, stream);
-  for (size_t i = 0; i < n; i++) {
-    const float* a = &acc[i * B2C_EVIDENCE_STRIDE];
-    float* e = &out[i * 7];
-    e[0] = a[0];
-    e[1] = a[1];
-    e[2] = a[2];
-    e[3] = a[7] > 0.f ? (a[0] * a[0]) / a[7] : 0.f;  // the participation ratio of the views' in-mask mass
-    e[4] = a[4];
-    e[5] = a[5];
-    e[6] = a[6];
+  if (g_evidence.count < n * B2C_EVIDENCE_STRIDE || n == 0) {
+    std::fill(out, out + n * 7, 0.f);
+    return;
   }
+  LAUNCH_CHECK(b2c_hip_evidence_export(m.n, g_evidence.ptr, g_evidence_rows.ptr, stream));
+  HIP_CHECK(hipMemcpyAsync(out, g_evidence_rows.ptr, n * 7 * sizeof(float), hipMemcpyDeviceToHost, stream));
+  HIP_CHECK(hipStreamSynchronize(stream));
+}
+
+void download_labels(const Model& m, float* out, hipStream_t stream) {
+  const size_t n = (size_t)m.n;
+  if (!g_labels_valid || g_labels.count < n * B2C_LABEL_BINS || n == 0) {
+    std::fill(out, out + n * 2, 0.f);
+    return;
+  }
+  LAUNCH_CHECK(b2c_hip_label_export(m.n, g_labels.ptr, g_label_rows.ptr, stream));
+  HIP_CHECK(hipMemcpyAsync(out, g_label_rows.ptr, n * 2 * sizeof(float), hipMemcpyDeviceToHost, stream));
+  HIP_CHECK(hipStreamSynchronize(stream));
+}
+
+std::vector<float> download_evidence(const Model& m, hipStream_t stream) {
+  std::vector<float> out((size_t)m.n * 7);
+  download_evidence(m, out.data(), stream);
   return out;
 }
 
 std::vector<float> download_labels(const Model& m, hipStream_t stream) {
-  const size_t n = (size_t)m.n;
-  std::vector<float> out(n * 2, 0.f);
-  if (!g_labels_valid || g_labels.count < n * B2C_LABEL_BINS || n == 0) return out;
-  const std::vector<float> acc = g_labels.download(n * B2C_LABEL_BINS, stream);
-  for (size_t i = 0; i < n; i++) {
-    const float* a = &acc[i * B2C_LABEL_BINS];
-    float total = 0.f, best = 0.f;
-    int win = 0;
-    for (int k = 0; k < B2C_LABEL_BINS; k++) {  // the first class with the largest vote wins
-      total += a[k];
-      if (a[k] > best) {
-        best = a[k];
-        win = k;
-      }
-    }
-    if (total > 0.f) {
-      out[i * 2] = (float)win;
-      out[i * 2 + 1] = best / total;
-    }
-  }
+  std::vector<float> out((size_t)m.n * 2);
+  download_labels(m, out.data(), stream);
   return out;
 }
 

@@ -31,10 +31,12 @@ void compute_evidence(RenderCtx& ctx, const Model& m, const std::vector<ViewGPU>
 }
 // [n][7]: views = (sum w_in)^2 / sum w_in^2, the effective number of supporting views (evidence.cu:236-249).
 std::vector<float> download_evidence(const Model& m, hipStream_t stream);
+void download_evidence(const Model& m, float* out, hipStream_t stream);  // into the caller's host array
 // The device accumulator of the last compute_evidence: [n][*stride], w_all at offset 1.
 const float* evidence_device(int* stride);
 // [n][2] = (winning class id, its share of the splat's vote); both 0 for a splat no labelled view rendered.
 std::vector<float> download_labels(const Model& m, hipStream_t stream);
+void download_labels(const Model& m, float* out, hipStream_t stream);
 
 // Per-pixel depth distribution of the composited splats after project_splats + bin_and_sort
 // (probe.h:6-11): out[pix] = (accumulated alpha, first-surface depth at alpha tau (tau <= 0: the

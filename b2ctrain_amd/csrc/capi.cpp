@@ -437,17 +437,11 @@ int b2c_compute_evidence(b2c_ctx* c, const b2c_model* m, const b2c_view* const* 
 }
 
 int b2c_download_evidence(const b2c_model* m, float* out) {
-  return guarded([&] {
-    const std::vector<float> e = b2c::download_evidence(m->m, nullptr);
-    std::copy(e.begin(), e.end(), out);
-  });
+  return guarded([&] { b2c::download_evidence(m->m, out, nullptr); });
 }
 
 int b2c_download_labels(const b2c_model* m, float* out) {
-  return guarded([&] {
-    const std::vector<float> l = b2c::download_labels(m->m, nullptr);
-    std::copy(l.begin(), l.end(), out);
-  });
+  return guarded([&] { b2c::download_labels(m->m, out, nullptr); });
 }
 
 int b2c_probe_depth(b2c_ctx* c, float tau, float delta, const float* ref_z, float margin, float* out) {

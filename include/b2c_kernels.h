@@ -394,6 +394,13 @@ typedef struct b2c_evidence_sum_args {
 } b2c_evidence_sum_args;
 int b2c_hip_evidence_sum(const b2c_evidence_sum_args* a, hipStream_t stream);
 
+/* The rows of download_evidence / download_labels (evidence.cu:185-264) on the device, from the accumulators: out [n][7]
+ * (w_in, w_all, err, w_in^2 / sum w_in^2 or 0, dir xyz) from evidence [n][B2C_EVIDENCE_STRIDE]; out [n][2] (first class
+ * with the largest vote, its share; zeros without votes) from label_acc [n][B2C_LABEL_BINS]. The accumulators
+ * must be 16-byte aligned, the label rows 8-byte aligned. */
+int b2c_hip_evidence_export(int n, const float* evidence, float* out, hipStream_t stream);
+int b2c_hip_label_export(int n, const float* label_acc, float* out, hipStream_t stream);
+
 /* probe_kernel (probe.cu:7-53) after projection and binning: out[pix] = (accumulated alpha, the depth where it
  * first reaches tau (tau <= 0: the alpha-weighted mean depth, +inf under 5% coverage), the weight from more
  * than delta behind that depth, the weight from more than margin behind ref_z (NULL: none)). */
