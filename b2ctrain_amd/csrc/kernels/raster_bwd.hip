@@ -14,6 +14,8 @@
 #include "b2c_kernels.h"
 #include "raster_common.h"
 
+#include <type_traits>
+
 namespace b2c {
 namespace dev {
 namespace {
@@ -313,13 +315,20 @@ __device__ __forceinline__ void load8(const float* p, float* x) {
 // product: refine, fp16 only), with hi/lo fp16 splits so ~22 bits of the fp32 inputs survive. The opacity lane needs
 // no product of its own: where a fragment is unclamped v_alpha * gauss = -v_sigma / opacity, and both are
 // zero where it is clamped, so g8 = -(sum v_sigma) / opacity.
+//
+// Where the time goes (variants with a part left out, 1M splats at 1080p, 360 us): the replay's arithmetic 117 us (36 of
+// it the refine statistic), the reduction 105 us (per group 48 VALU of hi/lo splits, 8 MFMA of 16.5 cycles that
+// do not overlap the VALU, 6 LDS reads), the rows' stores 18 us, the rest staging, LDS writes and waits. The LDS is busy
+// 57% of the kernel. Leaving the alpha cap out of groups that cannot reach it and loading a batch's ids one batch
+// ahead (one dependent round trip less per batch): 370 -> 353 us; 98 -> 90 us on 100k splats at 800x800, 747 -> 705 us
+// on a dense slab of 3M. Loading the records ahead too costs 14 registers and a wave: 398 us.
 template <bool FEAT, bool HOLLOW>
 __global__ void __launch_bounds__(64) raster_bwd_mfma_kernel(b2c_raster_bwd_args a) {
   constexpr bool EXT = FEAT || HOLLOW;
   constexpr int ROW = ROW_FLOATS<FEAT>;
   __shared__ float4 s_g0[BATCH];   // (D, E, F, c00 / 2): sigma_coefs at this tile
-  __shared__ float4 s_g1[BATCH];   // (c01, c11 / 2, power, log2 opacity)
-  __shared__ float4 s_col[BATCH];  // (max(r, 0), max(g, 0), max(b, 0), sign bits of r, g, b)
+  __shared__ float4 s_g1[BATCH];   // (c01, c11 / 2, power, E H / W)
+  __shared__ float4 s_col[BATCH];  // (max(r, 0), max(g, 0), max(b, 0), log2 opacity)
   __shared__ float4 s_ext[EXT ? BATCH : 1];  // (feature xyz, camera depth)
   __shared__ uint32_t s_slot[BATCH];
   __shared__ __attribute__((aligned(16))) float sS[2 * G][SROW];  // rows 0-7 vis, 8-15 v_sigma
@@ -345,10 +354,11 @@ __global__ void __launch_bounds__(64) raster_bwd_mfma_kernel(b2c_raster_bwd_args
   const float u = lx + 0.5f - RT_W * 0.5f, v = ly + 0.5f - RT_W * 0.5f;  // offset from the tile centre
   const float tcx = tx * RT_W + RT_W * 0.5f, tcy = ty * RT_W + RT_W * 0.5f;
   const PixelPoly pp = pixel_poly(u, v);
-  const float u2 = u + u, v2 = v + v;
   PixelState ps = load_pixel<FEAT, HOLLOW>(a, px, py, range.x, compact ? a.clast : a.last_idx);
-  // refine: sqrt(W^2 gx^2 + H^2 gy^2) = W sqrt(gx^2 + rho gy^2), W folded into the per-pixel scale
-  const float rho = ((float)a.H * (float)a.H) / ((float)a.W * (float)a.W);
+  // refine: sqrt(W^2 gx^2 + H^2 gy^2) = W sqrt(gx^2 + (gy H / W)^2), W folded into the per-pixel scale and H / W
+  // into gy's terms (the sigma gradient 2a u + b v + D, b u + 2c v + E)
+  const float hw = (float)a.H / (float)a.W;
+  const float u2 = u + u, v2h = (v + v) * hw, uh = u * hw;
   const float r_scale = ps.inv_final_a * R_SCALE * (float)a.W;
   const float cv_x = ps.vo.x, cv_y = ps.vo.y, cv_z = ps.vo.z;
 
@@ -374,20 +384,31 @@ __global__ void __launch_bounds__(64) raster_bwd_mfma_kernel(b2c_raster_bwd_args
   float Q = -ps.v_o_w;  // sum over composited splats behind of (colour . v_rgb) * vis, minus the v_o_w term
   float Sh = 0.f;       // HOLLOW: sum over composited splats behind of vis * penalty
   const bool live_px = ps.inside;
+  // the ids and emit positions of the next batch are loaded while this one is replayed
+  uint32_t nxt_id = 0, nxt_slot = 0;
+  {
+    const uint32_t first = range.y > range.x + BATCH ? range.y - BATCH : range.x;
+    if (lane < (int)(range.y - first)) {
+      nxt_id = list_vals[first + lane];
+      nxt_slot = list_slots[first + lane];
+    }
+  }
   for (uint32_t batch_end = range.y; batch_end > range.x;) {
     const uint32_t batch_start = batch_end > range.x + BATCH ? batch_end - BATCH : range.x;
     const int count = (int)(batch_end - batch_start);
     __syncthreads();
     const int ngroups = (count + G - 1) / G;
+    bool may_clamp = false;
     if (lane < count) {
-      const uint32_t gid = list_vals[batch_start + lane];
-      s_slot[lane] = list_slots[batch_start + lane];
+      const uint32_t gid = nxt_id;
+      s_slot[lane] = nxt_slot;
       const float4* rec = reinterpret_cast<const float4*>(a.raster_rec) + (size_t)gid * 4;
       const float4 r0 = rec[0], r1 = rec[1], r2 = rec[2];
       const float3 def = sigma_coefs(r0.x, r0.y, r0.z, r0.w, r1.x, tcx, tcy);
       s_g0[lane] = make_float4(def.x, def.y, def.z, r0.z);
-      s_g1[lane] = make_float4(r0.w, r1.x, r1.z, r2.w);
-      s_col[lane] = make_float4(r2.x, r2.y, r2.z, r1.w);
+      s_g1[lane] = make_float4(r0.w, r1.x, r1.z, def.y * hw);
+      s_col[lane] = r2;
+      may_clamp = clamp_possible(r0.x, r0.y, r0.z, r0.w, r1.x, r2.w, tcx, tcy);
       if constexpr (EXT) s_ext[lane] = rec[3];
     } else if (lane < ngroups * G) {  // pad the last group with null splats, never composited: power = 0
       s_g0[lane] = make_float4(0.f, 0.f, 1.f, 0.f);  // and sigma = F = 1
@@ -395,6 +416,14 @@ __global__ void __launch_bounds__(64) raster_bwd_mfma_kernel(b2c_raster_bwd_args
       s_col[lane] = make_float4(0.f, 0.f, 0.f, 0.f);
       if constexpr (EXT) s_ext[lane] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
+    {
+      const uint32_t before = batch_start > range.x + BATCH ? batch_start - BATCH : range.x;
+      if (lane < (int)(batch_start - before)) {
+        nxt_id = list_vals[before + lane];
+        nxt_slot = list_slots[before + lane];
+      }
+    }
+    const uint64_t clamps = ballot64(may_clamp);  // the batch's splats that may reach the alpha cap
     __syncthreads();
     for (int grp = ngroups - 1; grp >= 0; grp--) {
       const int gbase = grp * G;
@@ -409,53 +438,54 @@ __global__ void __launch_bounds__(64) raster_bwd_mfma_kernel(b2c_raster_bwd_args
       const char* lds_ext = reinterpret_cast<const char*>(s_ext) + goff;
       // the last list index of the group this pixel composited, relative to the group start
       const int last_rel = (int)ps.last - (int)(batch_start + (uint32_t)gbase);
-#pragma unroll
-      for (int jj = G - 1; jj >= 0; jj--) {
-        float o_vis = 0.f, o_vs = 0.f, o_r = 0.f;
-        {
-          const float4 g0 = *reinterpret_cast<const float4*>(lds_g0 + jj * 16);
-          const float4 g1 = *reinterpret_cast<const float4*>(lds_g1 + jj * 16);
-          const float sigma = poly_sigma(g0.w, g1.x, g1.y, g0.x, g0.y, g0.z, pp);
-          // the forward's test: sigma <= power (a NaN sigma fails)
-          const bool in = live_px & (jj < last_rel) & (sigma <= g1.z);
-          {  // straight-line: a lane without this fragment computes zeros (alpha = 0)
-            // a lane without this fragment runs the same arithmetic with alpha = 0: ra = 1, vis = 0,
-            // v_sigma = 0 and T, Q unchanged (every operand stays finite)
-            const float araw = fragment_alpha(sigma, g1.w);
-            const float alpha = in ? fminf(ALPHA_MAX, araw) : 0.f;
-            const float ra = __builtin_amdgcn_rcpf(1.f - alpha);
-            const float Tb = T * ra;
-            const float vis = alpha * Tb;
-            const float4 col = *reinterpret_cast<const float4*>(lds_col + jj * 16);
-            float cv = col.x * cv_x + col.y * cv_y + col.z * cv_z;
-            float4 ext = make_float4(0.f, 0.f, 0.f, 0.f);
-            if constexpr (EXT) ext = *reinterpret_cast<const float4*>(lds_ext + jj * 16);
-            if constexpr (FEAT) cv = cv + (ext.x * ps.vf.x + ext.y * ps.vf.y + ext.z * ps.vf.z);
-            const float v_alpha_photo = Tb * cv - ra * Q;
-            float v_alpha = v_alpha_photo, hh = 0.f;
-            if constexpr (HOLLOW) {
-              hh = hollow_h(ext.w, ps.href);
-              v_alpha = v_alpha + a.hollow_lam * (Tb * hh - ra * Sh);
-            }
-            const bool unclamped = araw <= ALPHA_MAX;  // clamped: no sigma gradient
-            const float v_sigma = unclamped ? -alpha * v_alpha : 0.f;
-            // refine statistic: |d(loss)/d(mean2d)| scaled to pixels, over the final alpha, from the
-            // photometric (and feature) terms only
-            const float v_sigma_photo = HOLLOW ? (unclamped ? -alpha * v_alpha_photo : 0.f) : v_sigma;
-            // the sigma gradient in pixels: 2a u + b v + D, b u + 2c v + E
-            const float gx = __builtin_fmaf(g0.w, u2, __builtin_fmaf(g1.x, v, g0.x));
-            const float gy = __builtin_fmaf(g1.x, u, __builtin_fmaf(g1.y, v2, g0.y));
-            o_r = fabsf(v_sigma_photo) * __builtin_amdgcn_sqrtf(gx * gx + rho * gy * gy) * r_scale;
-            o_vis = vis;
-            o_vs = v_sigma;
-            T = Tb;
-            Q = Q + vis * cv;
-            if constexpr (HOLLOW) Sh = Sh + vis * hh;
-          }
+      // One fragment, straight-line: a lane without it (past its last entry, or sigma above the cutoff; a NaN sigma
+      // fails) runs the same arithmetic with alpha = 0: ra = 1, vis = 0, v_sigma = 0 and T, Q unchanged (every
+      // operand stays finite). CAP: some splat of the group may reach the alpha cap, so alpha is capped and a capped
+      // fragment has no sigma gradient; a group without one, nearly every group, leaves those three operations
+      // out and computes the same values.
+      const auto replay = [&](auto cap, int jj) {
+        constexpr bool CAP = decltype(cap)::value;
+        const float4 g0 = *reinterpret_cast<const float4*>(lds_g0 + jj * 16);
+        const float4 g1 = *reinterpret_cast<const float4*>(lds_g1 + jj * 16);
+        const float4 col = *reinterpret_cast<const float4*>(lds_col + jj * 16);
+        const float sigma = poly_sigma(g0.w, g1.x, g1.y, g0.x, g0.y, g0.z, pp);
+        const bool in = live_px & (jj < last_rel) & (sigma <= g1.z);  // the forward's test
+        const float araw = fragment_alpha(sigma, col.w);
+        const float alpha = in ? (CAP ? fminf(ALPHA_MAX, araw) : araw) : 0.f;
+        const float ra = __builtin_amdgcn_rcpf(1.f - alpha);
+        const float Tb = T * ra;
+        const float vis = alpha * Tb;
+        float cv = col.x * cv_x + col.y * cv_y + col.z * cv_z;
+        float4 ext = make_float4(0.f, 0.f, 0.f, 0.f);
+        if constexpr (EXT) ext = *reinterpret_cast<const float4*>(lds_ext + jj * 16);
+        if constexpr (FEAT) cv = cv + (ext.x * ps.vf.x + ext.y * ps.vf.y + ext.z * ps.vf.z);
+        const float v_alpha_photo = Tb * cv - ra * Q;
+        float v_alpha = v_alpha_photo, hh = 0.f;
+        if constexpr (HOLLOW) {
+          hh = hollow_h(ext.w, ps.href);
+          v_alpha = v_alpha + a.hollow_lam * (Tb * hh - ra * Sh);
         }
-        sS[jj][lane] = o_vis;
-        sS[G + jj][lane] = o_vs;
-        sR[jj][lane] = pk_rtz(o_r, 0.f).x;
+        const bool free = !CAP | (araw <= ALPHA_MAX);
+        const float v_sigma = free ? -alpha * v_alpha : 0.f;
+        // refine statistic: |d(loss)/d(mean2d)| scaled to pixels, over the final alpha, from the photometric
+        // (and feature) terms only
+        const float v_sigma_photo = HOLLOW ? (free ? -alpha * v_alpha_photo : 0.f) : v_sigma;
+        const float gx = __builtin_fmaf(g0.w, u2, __builtin_fmaf(g1.x, v, g0.x));
+        const float gy = __builtin_fmaf(g1.x, uh, __builtin_fmaf(g1.y, v2h, g1.w));
+        const float refine = fabsf(v_sigma_photo) * __builtin_amdgcn_sqrtf(__builtin_fmaf(gy, gy, gx * gx)) * r_scale;
+        T = Tb;
+        Q = Q + vis * cv;
+        if constexpr (HOLLOW) Sh = Sh + vis * hh;
+        sS[jj][lane] = vis;
+        sS[G + jj][lane] = v_sigma;
+        sR[jj][lane] = pk_rtz(refine, 0.f).x;
+      };
+      if ((clamps >> gbase) & ((1u << G) - 1u)) {  // wave-uniform
+#pragma unroll
+        for (int jj = G - 1; jj >= 0; jj--) replay(std::true_type{}, jj);
+      } else {
+#pragma unroll
+        for (int jj = G - 1; jj >= 0; jj--) replay(std::false_type{}, jj);
       }
       __syncthreads();
       // ---- reduction over the 64 pixels on MFMA

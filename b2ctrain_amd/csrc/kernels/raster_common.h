@@ -180,6 +180,18 @@ __device__ __forceinline__ uint32_t quadrant_mask(float mx, float my, float ah, 
   return mask;
 }
 
+// Whether a fragment of this splat in the tile could reach the alpha cap: log2 alpha is log2 opacity - sigma
+// log2 e, and sigma, 0 or more exactly, rounds no further below 0 than 1e-5 of the quadratic's term magnitudes
+// over the tile (quadrant_mask's bound). -0.0015 lies below log2 0.999 by 30 roundings of the exponent. Anything
+// not finite counts as possible.
+__device__ __forceinline__ bool clamp_possible(float mx, float my, float ah, float b, float ch, float log2_op, float tcx,
+                                               float tcy) {
+  const float mxr = fabsf(mx - tcx), myr = fabsf(my - tcy), bb = fabsf(b);
+  const float scale = ((ah * mxr + bb * myr) * mxr + ch * myr * myr) +
+                      3.5f * ((2.f * ah + bb) * mxr + (bb + 2.f * ch) * myr) + 12.25f * (ah + bb + ch);
+  return !(log2_op + (1e-5f * LOG2E) * scale < -0.0015f);
+}
+
 // DPP controls (GCN/CDNA): row_shr:n = 0x110 + n, row_ror:n = 0x120 + n, row_bcast:15 = 0x142,
 // row_bcast:31 = 0x143, wave_shl:1 = 0x130, wave_shr:1 = 0x138. Lanes whose source is outside the row mask or
 // the wave get `fill`.
