@@ -395,12 +395,12 @@ __device__ __forceinline__ uint32_t select_bit64(uint32_t lo, uint32_t hi, uint3
 
 // Small splats: each wave takes 64 consecutive depth ranks, whose slot ranges [tile_off - count, tile_off)
 // are adjacent (big splats' ranges, filled by emit_big_kernel, interleave). The wave's intersections are
-// dealt to the lanes round-robin: intersection q belongs to the last rank whose running start is <= q (a
-// binary search over the wave's 64 starts in LDS) and is the k-th set bit of that splat's hit mask
-// (row-major bbox order; a bbox of up to 64 tiles: the mask of hit_info or of hit_wide). Every lane does
+// dealt to the lanes round-robin: intersection q belongs to the last rank whose running start is <= q
+// (slot_owner) and is the k-th set bit of that splat's hit mask (row-major bbox order; a bbox of up to 64 tiles: the mask of hit_info or of hit_wide). Every lane does
 // the same work and consecutive lanes write consecutive slots. Big splats only record their base.
 __global__ void __launch_bounds__(256) emit_small_kernel(b2c_emit_args a, uint32_t* __restrict__ big_base) {
-  __shared__ uint32_t s_start[4][64], s_base[4][64], s_mask[4][64], s_mask_hi[4][64], s_info[4][64], s_id[4][64];
+  __shared__ uint32_t s_own[4][64], s_start[4][64], s_base[4][64], s_mask[4][64], s_mask_hi[4][64], s_info[4][64], s_id[4][64],
+      s_inv[4][64];
   const int w = threadIdx.x >> 6, lane = lane_id();
   const int r = blockIdx.x * 256 + threadIdx.x;
   uint32_t i = 0, cnt = 0, base = 0;
@@ -429,18 +429,18 @@ __global__ void __launch_bounds__(256) emit_small_kernel(b2c_emit_args a, uint32
   s_mask[w][lane] = wide.x;
   s_mask_hi[w][lane] = wide.y;
   s_info[w][lane] = hi.y;
+  s_inv[w][lane] = 32768u / max(hi.y >> 24, 1u) + 1u;  // bit / width = (bit * this) >> 15 for bits and widths up to 64
   s_id[w][lane] = i;
-  __syncthreads();
-  for (uint32_t q = (uint32_t)lane; q < total; q += 64u) {
-    int j = 0;  // last lane with start <= q (the lanes after the owner start past q)
-#pragma unroll
-    for (int step = 32; step >= 1; step >>= 1)
-      if (s_start[w][j + step] <= q) j += step;
+  wave_lds_fence();  // read by their own wave
+  for (uint32_t q0 = 0; q0 < total; q0 += 64u) {
+    const uint32_t j = slot_owner(s_own[w], incl - c, c, q0, lane);
+    const uint32_t q = q0 + (uint32_t)lane;
+    if (q >= total) break;  // in the last step only
     const uint32_t k = q - s_start[w][j];
     const uint32_t info = s_info[w][j];
     const uint32_t min_x = info & 0xFFFu, min_y = (info >> 12) & 0xFFFu, bw = info >> 24;
     const uint32_t bit = select_bit64(s_mask[w][j], s_mask_hi[w][j], k);
-    const uint32_t row = bit / bw;
+    const uint32_t row = (bit * s_inv[w][j]) >> 15;
     const uint32_t slot = s_base[w][j] + k;
     a.keys[slot] = (min_y + row) * (uint32_t)a.tiles_x + min_x + (bit - row * bw);
     a.vals[slot] = s_id[w][j];
@@ -478,20 +478,22 @@ __global__ void __launch_bounds__(256) emit_big_kernel(b2c_emit_args a, const ui
     // the record is used here, so its loads share the third round trip (instead of being sunk into the
     // tile loop's guard)
     asm volatile("" : : "v"(g.mx), "v"(g.my), "v"(g.conic.c00), "v"(g.conic.c01), "v"(g.conic.c11), "v"(g.power));
+    const TileTest by = TileTest::of(g.conic);
     const bool fits = base + cnt <= a.cap;
     const uint32_t begin = k * info.w, end = fits ? min(begin + info.w, info.z) : begin;
     const uint32_t off_end = fits ? (end < info.z ? off_next : cnt) : off;
-    const int min_x = (int)(info.x & 0xFFFFu), min_y = (int)(info.x >> 16), bw = (int)info.y;
+    const int min_x = (int)(info.x & 0xFFFFu), min_y = (int)(info.x >> 16);
+    const BoxRows rows = BoxRows::of(info.y, info.z);
     uint32_t written = off;
     for (uint32_t b0 = begin; b0 < end; b0 += 64) {
       const uint32_t b = b0 + (uint32_t)lane;
       bool h = false;
       int tx = 0, ty = 0;
       if (b < end) {
-        tx = min_x + (int)(b % (uint32_t)bw);
-        ty = min_y + (int)(b / (uint32_t)bw);
-        const float rx = tx * (float)RT_W, ry = ty * (float)RT_W;
-        h = tile_hit(rx, ry, rx + RT_W, ry + RT_W, g.mx, g.my, g.conic, g.power);
+        const uint32_t row = rows.row(b);
+        tx = min_x + (int)(b - row * rows.bw);
+        ty = min_y + (int)row;
+        h = tile_hit(tx * (float)RT_W, ty * (float)RT_W, g.mx, g.my, g.conic, g.power, by);
       }
       const uint64_t mk = ballot64(h);
       if (h) {

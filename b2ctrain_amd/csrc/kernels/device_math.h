@@ -104,24 +104,60 @@ __device__ __forceinline__ float calc_sigma(float px, float py, float c00, float
 }
 
 // Ellipse-vs-rectangle test (StopThePop / brush `will_primitive_contribute`, splat_math.cuh:27-41): the
-// rectangle point nearest the centre along each edge in the conic metric must satisfy sigma <= power.
-__device__ __forceinline__ bool tile_hit(float rmin_x, float rmin_y, float rmax_x, float rmax_y, float mx, float my,
-                                         Sym2 conic, float power) {
+// rectangle point nearest the centre along each edge in the conic metric must satisfy sigma <= power. The
+// rectangle is a raster tile, (rmin_x, rmin_y) its corner.
+//
+// The reference's edge parameter is t = (dx c00 ex + dx c01 ey) / (dx c00 dx) with dx = +-8 the edge and e the
+// centre's offset from the corner, clamped to [0, 1], and the point is the corner + t dx. Scaling by 8 is exact,
+// so the same value, bit for bit, is the quotient q = (c00 ex + c01 ey) / c00 clamped to the edge, [0, 8] or
+// [-8, 0]. The quotient comes from the splat's reciprocal r = 1 / c00: with r correctly rounded,
+// q0 = n r and q = q0 + (n - c00 q0) r round to the IEEE quotient (P. Markstein, "Computation of elementary
+// functions on the IBM RISC System/6000 processor", 1990) while nothing underflows: TileTest::of keeps to
+// conics in [2^-40, 2^40] and leaves others, splats over a million pixels wide, to the division. 38 instead of 62
+// operations a test.
+struct TileTest {
+  float r00, r11;  // 1 / c00, 1 / c11, or 0: divide
+  __device__ __forceinline__ static float rcp_or_0(float c) { return c >= 0x1p-40f && c <= 0x1p40f ? 1.f / c : 0.f; }
+  __device__ __forceinline__ static TileTest of(Sym2 conic) { return TileTest{rcp_or_0(conic.c00), rcp_or_0(conic.c11)}; }
+};
+
+__device__ __forceinline__ float quotient(float n, float c, float r) {
 #pragma clang fp contract(off)
-  bool x_left = mx < rmin_x, x_right = mx > rmax_x, in_x = !(x_left || x_right);
-  bool y_above = my < rmin_y, y_below = my > rmax_y, in_y = !(y_above || y_below);
-  if (in_x && in_y) return true;
-  float corner_x = x_left ? rmin_x : rmax_x, corner_y = y_above ? rmin_y : rmax_y;
-  float width = rmax_x - rmin_x, height = rmax_y - rmin_y;
-  float dxf = x_left ? width : -width, dyf = y_above ? height : -height;
-  float diff_x = mx - corner_x, diff_y = my - corner_y;
-  float tx_raw = (dxf * conic.c00 * diff_x + dxf * conic.c01 * diff_y) / (dxf * conic.c00 * dxf);
-  float ty_raw = (dyf * conic.c01 * diff_x + dyf * conic.c11 * diff_y) / (dyf * conic.c11 * dyf);
-  float tx = in_y ? 0.f : fminf(fmaxf(tx_raw, 0.f), 1.f);
-  float ty = in_x ? 0.f : fminf(fmaxf(ty_raw, 0.f), 1.f);
-  float px = corner_x + tx * dxf, py = corner_y + ty * dyf;
-  return calc_sigma(px, py, conic.c00, conic.c01, conic.c11, mx, my) <= power;
+  if (r == 0.f) return n / c;
+  const float q0 = n * r;
+  return __builtin_fmaf(__builtin_fmaf(-c, q0, n), r, q0);
 }
+
+__device__ __forceinline__ bool tile_hit(float rmin_x, float rmin_y, float mx, float my, Sym2 conic, float power,
+                                         TileTest by) {
+#pragma clang fp contract(off)
+  const float rmax_x = rmin_x + RT_W, rmax_y = rmin_y + RT_W;
+  const bool x_left = mx < rmin_x, x_right = mx > rmax_x, in_x = !(x_left | x_right);
+  const bool y_above = my < rmin_y, y_below = my > rmax_y, in_y = !(y_above | y_below);
+  const float corner_x = x_left ? rmin_x : rmax_x, corner_y = y_above ? rmin_y : rmax_y;
+  const float ex = mx - corner_x, ey = my - corner_y;
+  const float lo_x = x_left ? 0.f : -(float)RT_W, lo_y = y_above ? 0.f : -(float)RT_W;
+  const float qx = quotient(conic.c00 * ex + conic.c01 * ey, conic.c00, by.r00);
+  const float qy = quotient(conic.c01 * ex + conic.c11 * ey, conic.c11, by.r11);
+  const float px = corner_x + (in_y ? 0.f : fminf(fmaxf(qx, lo_x), lo_x + RT_W));
+  const float py = corner_y + (in_x ? 0.f : fminf(fmaxf(qy, lo_y), lo_y + RT_W));
+  const bool edge = calc_sigma(px, py, conic.c00, conic.c01, conic.c11, mx, my) <= power;
+  return (in_x & in_y) | edge;
+}
+
+// Row and column of a bounding box's tile number, for boxes of any width: in a box of at most 2^20 tiles the row is
+// (b + 1/2) / width by one multiplication, truncated: the fraction stays 1 / (2 width) away from the integers and
+// the product is off by less than 2 rows 2^-24. Larger boxes divide (the integer division is 18 operations).
+struct BoxRows {
+  uint32_t bw;
+  float inv;  // 0: divide
+  __device__ __forceinline__ static BoxRows of(uint32_t bw, uint32_t area) {
+    return BoxRows{bw, area <= (1u << 20) ? 1.f / (float)bw : 0.f};
+  }
+  __device__ __forceinline__ uint32_t row(uint32_t b) const {
+    return inv != 0.f ? (uint32_t)(((float)b + 0.5f) * inv) : b / bw;
+  }
+};
 
 struct TileBox { int min_x, min_y, max_x, max_y; };
 
@@ -295,6 +331,37 @@ __device__ __forceinline__ uint32_t popc64(uint64_t m) { return (uint32_t)__popc
 // Number of set bits of m strictly below this lane.
 __device__ __forceinline__ uint32_t mbcnt64(uint64_t m) {
   return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+
+// Work shared out over a wave: lane j owns the slots [start_j, start_j + count_j) (starts ascending, the exclusive
+// prefix of the counts). The owner of slot t0 + lane, for the 64 slots from t0: each owner with slots here marks
+// its first one in `own` (64 words of LDS of this wave), and a running maximum over the lanes (DPP row shifts and
+// broadcasts) carries the mark forward. A binary search over the starts, which it replaces, is six dependent LDS
+// reads. Every lane of the wave must call it.
+__device__ __forceinline__ void wave_lds_fence() {  // LDS operations of a wave complete in order
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+template <int CTRL, int ROW_MASK>
+__device__ __forceinline__ uint32_t dpp_or_0(uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, ROW_MASK, 0xF, false);
+}
+
+__device__ __forceinline__ uint32_t slot_owner(uint32_t* own, uint32_t start, uint32_t count, uint32_t t0, int lane) {
+  own[lane] = 0u;
+  wave_lds_fence();
+  const uint32_t first = start > t0 ? start - t0 : 0u;
+  if (count != 0u && start + count > t0 && first < 64u) own[first] = (uint32_t)lane;
+  wave_lds_fence();
+  uint32_t o = own[lane];
+  wave_lds_fence();  // before the next call clears it
+  o = max(o, dpp_or_0<0x111, 0xF>(o));  // row_shr:1, 2, 4, 8
+  o = max(o, dpp_or_0<0x112, 0xF>(o));
+  o = max(o, dpp_or_0<0x114, 0xF>(o));
+  o = max(o, dpp_or_0<0x118, 0xF>(o));
+  o = max(o, dpp_or_0<0x142, 0xA>(o));  // row_bcast:15 into rows 1 and 3
+  return max(o, dpp_or_0<0x143, 0xC>(o));  // row_bcast:31 into rows 2 and 3
 }
 
 }  // namespace dev

@@ -20,11 +20,14 @@ namespace {
 constexpr int PROJ_BLOCK = 256;
 
 // Tile tests of the wave's small splats (bbox of at most 64 tiles) are shared out over all 64 lanes: the
-// splats' bbox areas are prefix-summed across the wave, test t goes to lane t mod 64, which finds the
-// owning splat by binary search over the prefix and sets the hit bit in the owner's mask in LDS. A wave
-// then costs ceil(sum of areas / 64) tile tests per lane instead of its largest bbox.
+// splats' bbox areas are prefix-summed across the wave and test t goes to lane t mod 64 (slot_owner names its
+// splat). The 64 results of a step are one ballot, from which each splat's lane shifts its own bits into its
+// mask. A wave then costs ceil(sum of areas / 64) tile tests per lane instead of its largest bbox. (A binary search
+// for the splat, LDS atomics for the mask bits and the divisions of the tile test: 120 against 113 us on 1M splats at
+// 1080p, 968 against 845 us on a dense slab of 3M, 475 against 388 us at 4K with large splats.)
 struct WaveRec {
   float mx, my, c00, c01, c11, power;
+  TileTest by;
   uint32_t origin;  // min_x | min_y << 16
   uint32_t bwm;     // bbox width (bits 0-15); a small splat's also (32768 / width + 1) << 16: bit / width =
                     // (bit * that) >> 15 for every bit < 64 (width <= 64: the error bit / 32768 stays below
@@ -56,8 +59,7 @@ __device__ __forceinline__ uint32_t big_nchunks(uint4 info) { return (info.z + i
 template <int DEG, bool HALF, bool FEAT>
 __global__ void __launch_bounds__(PROJ_BLOCK) project_kernel(b2c_project_args a) {
   __shared__ WaveRec s_rec[PROJ_BLOCK];
-  __shared__ uint32_t s_incl[PROJ_BLOCK];
-  __shared__ uint32_t s_mask[2][PROJ_BLOCK];  // hit mask bits 0-31, 32-63
+  __shared__ uint32_t s_start[PROJ_BLOCK], s_own[PROJ_BLOCK];
   const int i = blockIdx.x * PROJ_BLOCK + threadIdx.x;
   const int lane = lane_id();
   const int wbase = threadIdx.x & ~63;
@@ -89,11 +91,11 @@ __global__ void __launch_bounds__(PROJ_BLOCK) project_kernel(b2c_project_args a)
       small = !big;
       if (small) {
         area = (uint32_t)(bw * bh);
-        s_rec[threadIdx.x] = WaveRec{pr.px, pr.py, pr.conic.c00, pr.conic.c01, pr.conic.c11, power,
+        s_rec[threadIdx.x] = WaveRec{pr.px, pr.py, pr.conic.c00, pr.conic.c01, pr.conic.c11, power, TileTest::of(pr.conic),
                                      (uint32_t)bb.min_x | ((uint32_t)bb.min_y << 16), pack_small_bw(bw)};
       } else {  // big: the geometry as the emit reads it back from the raster record (halved diagonal)
-        s_rec[threadIdx.x] = WaveRec{pr.px, pr.py, 2.f * (0.5f * pr.conic.c00), pr.conic.c01,
-                                     2.f * (0.5f * pr.conic.c11), power,
+        const Sym2 conic{2.f * (0.5f * pr.conic.c00), pr.conic.c01, 2.f * (0.5f * pr.conic.c11)};
+        s_rec[threadIdx.x] = WaveRec{pr.px, pr.py, conic.c00, conic.c01, conic.c11, power, TileTest::of(conic),
                                      (uint32_t)bb.min_x | ((uint32_t)bb.min_y << 16), (uint32_t)bw};
       }
       // SH colour at the camera-to-splat direction (project.cu:44-55)
@@ -169,37 +171,33 @@ __global__ void __launch_bounds__(PROJ_BLOCK) project_kernel(b2c_project_args a)
     const uint32_t t = __shfl_up(incl, o);
     if (lane >= o) incl += t;
   }
-  const uint32_t total = __shfl(incl, 63);
-  s_incl[threadIdx.x] = incl;
-  s_mask[0][threadIdx.x] = 0u;
-  s_mask[1][threadIdx.x] = 0u;
-  __syncthreads();
+  const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+  const uint32_t start = incl - area;
+  s_start[threadIdx.x] = start;
+  wave_lds_fence();  // the records and starts are read by their own wave
+  uint64_t mask = 0;  // this lane's splat's hits, bits in row-major bbox order
   for (uint32_t t0 = 0; t0 < total; t0 += 64) {
+    const uint32_t owner = wbase + slot_owner(s_own + wbase, start, area, t0, lane);
     const uint32_t t = t0 + (uint32_t)lane;
+    bool hit = false;
     if (t < total) {
-      int lo = 0, hi = 63;  // owner: the first lane whose inclusive prefix exceeds t
-#pragma unroll
-      for (int step = 0; step < 6; step++) {
-        const int mid = (lo + hi) >> 1;
-        if (s_incl[wbase + mid] > t) hi = mid; else lo = mid + 1;
-      }
-      const int owner = lo;
-      const WaveRec rec = s_rec[wbase + owner];
-      const uint32_t prev = owner == 0 ? 0u : s_incl[wbase + owner - 1];
-      const uint32_t bit = t - prev;
+      const WaveRec rec = s_rec[owner];
+      const uint32_t bit = t - s_start[owner];
       const uint32_t bw = rec.bwm & 0xFFFFu;
       const uint32_t row = (bit * (rec.bwm >> 16)) >> 15;  // bit / bw
       const int tx = (int)(rec.origin & 0xFFFFu) + (int)(bit - row * bw);
       const int ty = (int)(rec.origin >> 16) + (int)row;
-      const float rx = tx * (float)RT_W, ry = ty * (float)RT_W;
-      if (tile_hit(rx, ry, rx + RT_W, ry + RT_W, rec.mx, rec.my, Sym2{rec.c00, rec.c01, rec.c11}, rec.power))
-        atomicOr(&s_mask[bit >> 5][wbase + owner], 1u << (bit & 31u));
+      hit = tile_hit(tx * (float)RT_W, ty * (float)RT_W, rec.mx, rec.my, Sym2{rec.c00, rec.c01, rec.c11}, rec.power, rec.by);
+    }
+    const uint64_t hits = ballot64(hit);
+    if (area != 0u && start < t0 + 64u && start + area > t0) {  // some of this splat's tests were among them
+      const uint64_t own = start >= t0 ? hits >> (start - t0) : hits << (t0 - start);
+      mask |= own & (~0ull >> (64u - area));
     }
   }
-  __syncthreads();
   if (small || big) {
     const uint32_t info = (uint32_t)bb.min_x | ((uint32_t)bb.min_y << 12) | ((uint32_t)(bb.max_x - bb.min_x) << 24);
-    const uint32_t lo = small ? s_mask[0][threadIdx.x] : 0u, hi = small ? s_mask[1][threadIdx.x] : 0u;
+    const uint32_t lo = small ? (uint32_t)mask : 0u, hi = small ? (uint32_t)(mask >> 32) : 0u;
     // The mask word of hit_info keeps the reference's meaning (binning.cu:37): the mask of a bbox of at
     // most 32 tiles, or 0xFFFFFFFF ("recompute"). A bbox of 33 to 64 tiles, or a full 32-tile mask (which
     // reads as "recompute"), keeps its mask in hit_wide; a big splat marks hit_wide (0, 0).
@@ -286,15 +284,17 @@ __global__ void __launch_bounds__(PROJ_BLOCK) project_kernel(b2c_project_args a)
       const uint32_t len = big_bbox_of_len(ar);
       const uint32_t k = q - s_cstart[lo];
       const uint32_t begin = k * len, end = min(begin + len, ar);
-      const int min_x = (int)(rec.origin & 0xFFFFu), min_y = (int)(rec.origin >> 16), rbw = (int)(rec.bwm & 0xFFFFu);
+      const int min_x = (int)(rec.origin & 0xFFFFu), min_y = (int)(rec.origin >> 16);
+      const BoxRows rows = BoxRows::of(rec.bwm & 0xFFFFu, ar);
       uint32_t hits = 0;
       for (uint32_t b0 = begin; b0 < end; b0 += 64) {
         const uint32_t b = b0 + (uint32_t)lane;
         bool h = false;
         if (b < end) {
-          const int tx = min_x + (int)(b % (uint32_t)rbw), ty = min_y + (int)(b / (uint32_t)rbw);
-          const float rx = tx * (float)RT_W, ry = ty * (float)RT_W;
-          h = tile_hit(rx, ry, rx + RT_W, ry + RT_W, rec.mx, rec.my, Sym2{rec.c00, rec.c01, rec.c11}, rec.power);
+          const uint32_t row = rows.row(b);
+          const int tx = min_x + (int)(b - row * rows.bw), ty = min_y + (int)row;
+          h = tile_hit(tx * (float)RT_W, ty * (float)RT_W, rec.mx, rec.my, Sym2{rec.c00, rec.c01, rec.c11}, rec.power,
+                       rec.by);
         }
         hits += popc64(ballot64(h));
       }
