@@ -6,8 +6,8 @@
 //   and ranks it round by round in input order (ballot "match" masks for the lanes below with the same
 //   digit, plus the wave's running per-digit count in LDS), so no block barrier sits inside the ranking
 //   loop; keys and values are staged in LDS sorted by digit and written out in runs. Every thread loads
-//   its KPT keys before it computes anything, so the loads of a tile are all in flight at once. KPT is 16
-//   for large sorts and 4 for small ones (enough workgroups to cover the chip).
+//   its keys before it computes anything, so the loads of a tile are all in flight at once. Tiles hold 8192 keys in
+//   large sorts and 2048 in small ones (enough workgroups to cover the chip); up to 4096 keys one workgroup sorts alone.
 // * Count scan: reduce-then-scan of tile_count gathered in depth order, four contiguous entries a thread;
 //   each workgroup of the second pass sums its predecessors' totals itself (no middle kernel).
 // * Emit: small splats one thread each over the set bits of their hit mask; splats whose bbox exceeds 64
@@ -23,11 +23,20 @@ namespace dev {
 namespace {
 
 constexpr int SORT_THREADS = 256;
-constexpr int KPT_BIG = 16;  // keys per thread of a large sort (4096-key tiles)
-constexpr int KPT_SMALL = 8;  // below BIG_SORT_MIN keys (2048-key tiles)
+// Keys per tile, in units of 256, and the threads that scatter one. A scatter workgroup's phases are chains of
+// LDS and barrier waits, so what counts is waves per CU: with 512 threads a tile and 16-bit digit counters a CU holds
+// 16 (8192-key tiles, 75 KB) or 32 of them. Against 256 threads and 32-bit counters, binning measured 3370 -> 2882 us
+// (127M intersections a view), 1640 -> 1304 us (62M at 4K, whose 9-bit pass held one workgroup per CU), 256 -> 237 us
+// (6M, 1M splats), 142 -> 132 us (0.9M, 100k splats). 1024 threads over 16384-key tiles: 3233 and 1550 us.
+constexpr int SCATTER_THREADS = 2 * SORT_THREADS;
+constexpr int KPT_SMALL = 8;   // 2048-key tiles
 constexpr uint32_t BIG_SORT_MIN = 1u << 22;
-constexpr int KPT_HUGE = 32;  // from HUGE_SORT_MIN keys (8192-key tiles)
+constexpr int KPT_BIG = 16;    // 4096-key tiles
+constexpr int KPT_HUGE = 32;   // 8192-key tiles, from HUGE_SORT_MIN keys
 constexpr uint32_t HUGE_SORT_MIN = 1u << 25;
+// Sorts of up to ONE_SORT_MAX keys (their number known to the host, one value array) run in one workgroup.
+constexpr int ONE_THREADS = 1024, ONE_KPT = 4;
+constexpr uint32_t ONE_SORT_MAX = ONE_THREADS * ONE_KPT;
 constexpr int RADIX = 256;
 constexpr int NWAVES = SORT_THREADS / 64;
 constexpr int SCAN_PER = 4;                         // count scan: contiguous entries per thread
@@ -59,7 +68,8 @@ __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v) {
   return v;
 }
 
-// Exclusive scan over a 256-thread block; returns the exclusive prefix, writes the block total.
+// Exclusive scan over a block of NW waves; returns the exclusive prefix, writes the block total.
+template <int NW = NWAVES>
 __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t* s_wsum, uint32_t& total) {
   const int w = threadIdx.x >> 6, l = lane_id();
   uint32_t inc = wave_incl_scan(v);
@@ -67,7 +77,7 @@ __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t* s_wsum
   __syncthreads();
   uint32_t wbase = 0, tot = 0;
 #pragma unroll
-  for (int k = 0; k < NWAVES; k++) {
+  for (int k = 0; k < NW; k++) {
     uint32_t s = s_wsum[k];
     if (k < w) wbase += s;
     tot += s;
@@ -186,21 +196,23 @@ __global__ void __launch_bounds__(SORT_THREADS) radix_scan_digits(uint32_t* __re
 // staging buffer sorted by digit, which is written out in order: each digit's keys of this tile form one
 // contiguous run in the output, so consecutive lanes write consecutive addresses. NV = 1 or 2 value arrays
 // ride along with the keys. R = 256 or 512 digits (8- or 9-bit passes); thread t owns digits t R/256 ...
-template <int NV, int KPT, int R>
-__global__ void __launch_bounds__(SORT_THREADS) radix_scatter(
+template <int NV, int KPT, int R, int TH>
+__global__ void __launch_bounds__(TH) radix_scatter(
     const uint32_t* __restrict__ keys_in, const uint32_t* __restrict__ vals_in, const uint32_t* __restrict__ vals2_in,
     uint32_t* __restrict__ keys_out, uint32_t* __restrict__ vals_out, uint32_t* __restrict__ vals2_out, uint32_t cap,
     const uint32_t* __restrict__ n_dev, int shift, int bits, const uint32_t* __restrict__ block_hist, uint32_t nblocks,
     const uint32_t* __restrict__ digit_total) {
-  constexpr uint32_t TILE = SORT_THREADS * KPT, CHUNK = 64 * KPT;
+  constexpr uint32_t TILE = TH * KPT, CHUNK = 64 * KPT;
+  constexpr int NW = TH / 64;
   __shared__ uint32_t s_key[TILE];
   __shared__ uint32_t s_val[TILE];  // one value array staged at a time (with NV = 2 the second follows the first)
-  constexpr int DPT = R / SORT_THREADS;  // digits per thread
+  constexpr int DPT = R > TH ? R / TH : 1;  // digits per thread (the threads past R have none)
+  const bool has_digits = threadIdx.x * DPT < R;
   // global position of the tile's first key of each digit minus its local (staging) offset: staging slot j
   // of digit d goes to s_gdelta[d] + j
   __shared__ uint32_t s_gdelta[R];
-  __shared__ uint32_t s_wcnt[NWAVES][R];
-  __shared__ uint32_t s_wsum[NWAVES];
+  __shared__ uint16_t s_wcnt[NW][R];  // counts and staging offsets, at most TILE
+  __shared__ uint32_t s_wsum[NW];
   const uint32_t tile = sort_tile(nblocks);
   if (tile >= nblocks) return;
   const uint32_t n = live_count(cap, n_dev);
@@ -224,33 +236,34 @@ __global__ void __launch_bounds__(SORT_THREADS) radix_scatter(
     uint32_t tot_d[DPT], mine[DPT], cnt[DPT], tot_sum = 0, cnt_sum = 0;
 #pragma unroll
     for (int j = 0; j < DPT; j++) {
-      const uint32_t d = threadIdx.x * DPT + j;
-      tot_d[j] = digit_total[d];
-      mine[j] = block_hist[(size_t)d * nblocks + tile];
-      const uint32_t next = tile + 1 < nblocks ? block_hist[(size_t)d * nblocks + tile + 1] : tot_d[j];
+      const uint32_t d = has_digits ? threadIdx.x * DPT + j : 0u;
+      tot_d[j] = has_digits ? digit_total[d] : 0u;
+      mine[j] = has_digits ? block_hist[(size_t)d * nblocks + tile] : 0u;
+      const uint32_t next = has_digits && tile + 1 < nblocks ? block_hist[(size_t)d * nblocks + tile + 1] : tot_d[j];
       cnt[j] = next - mine[j];
       tot_sum += tot_d[j];
       cnt_sum += cnt[j];
     }
     uint32_t tot;
-    uint32_t digit_start = block_excl_scan(tot_sum, s_wsum, tot);
-    uint32_t loff = block_excl_scan(cnt_sum, s_wsum, tot);
+    uint32_t digit_start = block_excl_scan<NW>(tot_sum, s_wsum, tot);
+    uint32_t loff = block_excl_scan<NW>(cnt_sum, s_wsum, tot);
 #pragma unroll
     for (int j = 0; j < DPT; j++) {
+      if (!has_digits) break;
       const uint32_t d = threadIdx.x * DPT + j;
       s_gdelta[d] = digit_start + mine[j] - loff;
       loff_d[j] = loff;
       digit_start += tot_d[j];
       loff += cnt[j];
 #pragma unroll
-      for (int k = 0; k < NWAVES; k++) s_wcnt[k][d] = 0u;
+      for (int k = 0; k < NW; k++) s_wcnt[k][d] = 0;
     }
   }
   __syncthreads();
   // 3. rank within the wave: rank = keys of the same digit earlier in this wave's stretch. All lanes read
   //    the running count before the round's leaders advance it (LDS instructions of a wave run in order).
   uint32_t rank[KPT];
-  uint32_t* wc = s_wcnt[w];
+  uint16_t* wc = s_wcnt[w];
 #pragma unroll
   for (int r = 0; r < KPT; r++) {
     const bool valid = w * CHUNK + (uint32_t)r * 64 + lane < tile_n;
@@ -258,19 +271,20 @@ __global__ void __launch_bounds__(SORT_THREADS) radix_scatter(
     const uint64_t peers = match_digit(d, bits, valid);
     const uint32_t lt = popc64(peers & lanemask_lt());
     const uint32_t before = wc[d];
-    if (valid && lt == 0) wc[d] = before + popc64(peers);
+    if (valid && lt == 0) wc[d] = (uint16_t)(before + popc64(peers));
     rank[r] = before + lt;
   }
   __syncthreads();
   // 4. per-wave counts become staging offsets
 #pragma unroll
   for (int j = 0; j < DPT; j++) {
+    if (!has_digits) break;
     const uint32_t d = threadIdx.x * DPT + j;
     uint32_t run = loff_d[j];
 #pragma unroll
-    for (int k = 0; k < NWAVES; k++) {
+    for (int k = 0; k < NW; k++) {
       const uint32_t c = s_wcnt[k][d];
-      s_wcnt[k][d] = run;
+      s_wcnt[k][d] = (uint16_t)run;
       run += c;
     }
   }
@@ -287,7 +301,7 @@ __global__ void __launch_bounds__(SORT_THREADS) radix_scatter(
   }
   __syncthreads();
   // 6. write out in digit runs
-  for (uint32_t j = threadIdx.x; j < tile_n; j += SORT_THREADS) {
+  for (uint32_t j = threadIdx.x; j < tile_n; j += TH) {
     const uint32_t k = s_key[j];
     const uint32_t g = s_gdelta[(k >> shift) & dmask] + j;
     keys_out[g] = k;
@@ -299,8 +313,93 @@ __global__ void __launch_bounds__(SORT_THREADS) radix_scatter(
     for (int r = 0; r < KPT; r++)
       if (w * CHUNK + (uint32_t)r * 64 + lane < tile_n) s_val[rank[r]] = val[1][r];
     __syncthreads();
-    for (uint32_t j = threadIdx.x; j < tile_n; j += SORT_THREADS) {
+    for (uint32_t j = threadIdx.x; j < tile_n; j += TH) {
       vals2_out[s_gdelta[(s_key[j] >> shift) & dmask] + j] = s_val[j];
+    }
+  }
+}
+
+// The whole sort of up to ONE_SORT_MAX keys in one workgroup: the passes of radix_scatter with keys and values in LDS
+// between them. Wave w owns entries [256 w, 256 w + 256) and ranks them in order; thread d < 256 turns digit d's
+// per-wave counts into staging offsets; 8-bit digits. Such a sort is bound by its chain of launches (12 for 32-bit
+// keys) and not by its keys: 37.5 -> 14.3 us at 64 keys, 37.9 -> 15.5 us at 1024, 41.7 -> 17.4 us at 4096; a whole
+// step over 1200 splats 261 -> 235 us.
+__global__ void __launch_bounds__(ONE_THREADS) sort_one_kernel(const uint32_t* __restrict__ keys_in,
+                                                               const uint32_t* __restrict__ vals_in,
+                                                               uint32_t* __restrict__ keys_out,
+                                                               uint32_t* __restrict__ vals_out, uint32_t n, int begin_bit,
+                                                               int end_bit) {
+  constexpr int NW = ONE_THREADS / 64;
+  constexpr uint32_t CHUNK = 64 * ONE_KPT;
+  __shared__ uint32_t s_key[ONE_SORT_MAX], s_val[ONE_SORT_MAX];
+  __shared__ uint16_t s_wcnt[NW][RADIX];
+  __shared__ uint32_t s_wsum[NW];
+  const int w = threadIdx.x >> 6, lane = lane_id();
+  const uint32_t first = w * CHUNK + (uint32_t)lane;
+  uint32_t key[ONE_KPT], val[ONE_KPT];
+#pragma unroll
+  for (int r = 0; r < ONE_KPT; r++) {
+    const uint32_t li = first + 64u * r;
+    key[r] = li < n ? keys_in[li] : 0u;
+    val[r] = li < n ? (vals_in ? vals_in[li] : li) : 0u;
+  }
+  for (int shift = begin_bit; shift < end_bit; shift += 8) {
+    const int bits = min(8, end_bit - shift);
+    const uint32_t dmask = (1u << bits) - 1u;
+    for (int t = threadIdx.x; t < NW * RADIX; t += ONE_THREADS) s_wcnt[t / RADIX][t % RADIX] = 0;
+    __syncthreads();
+    uint32_t rank[ONE_KPT];
+    uint16_t* wc = s_wcnt[w];
+#pragma unroll
+    for (int r = 0; r < ONE_KPT; r++) {
+      const bool valid = first + 64u * r < n;
+      const uint32_t d = (key[r] >> shift) & dmask;
+      const uint64_t peers = match_digit(d, bits, valid);
+      const uint32_t lt = popc64(peers & lanemask_lt());
+      const uint32_t before = wc[d];
+      if (valid && lt == 0) wc[d] = (uint16_t)(before + popc64(peers));
+      rank[r] = before + lt;
+    }
+    __syncthreads();
+    uint32_t cnt = 0u, tot;
+    if (threadIdx.x < RADIX) {
+#pragma unroll
+      for (int k = 0; k < NW; k++) cnt += s_wcnt[k][threadIdx.x];
+    }
+    uint32_t run = block_excl_scan<NW>(cnt, s_wsum, tot);
+    if (threadIdx.x < RADIX) {
+#pragma unroll
+      for (int k = 0; k < NW; k++) {
+        const uint32_t c = s_wcnt[k][threadIdx.x];
+        s_wcnt[k][threadIdx.x] = (uint16_t)run;
+        run += c;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < ONE_KPT; r++) {
+      if (first + 64u * r < n) {
+        const uint32_t lp = wc[(key[r] >> shift) & dmask] + rank[r];
+        s_key[lp] = key[r];
+        s_val[lp] = val[r];
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < ONE_KPT; r++) {
+      const uint32_t li = first + 64u * r;
+      if (li < n) {
+        key[r] = s_key[li];
+        val[r] = s_val[li];
+      }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < ONE_KPT; r++) {
+    const uint32_t li = first + 64u * r;
+    if (li < n) {
+      keys_out[li] = key[r];
+      vals_out[li] = val[r];
     }
   }
 }
@@ -598,14 +697,16 @@ void sort_pass(const uint32_t* src_k, const uint32_t* src_v, const uint32_t* src
                uint32_t* digit_total, hipStream_t stream) {
   const uint32_t nb = sort_blocks(n, KPT);
   const dim3 grid(8u * ((nb + 7u) / 8u));  // sort_tile's XCD-contiguous mapping
+  constexpr int TH = SCATTER_THREADS, K = KPT * SORT_THREADS / TH;
+  const dim3 block(TH);
   radix_upsweep<KPT, R><<<grid, dim3(SORT_THREADS), 0, stream>>>(src_k, n, n_dev, shift, bits, block_hist, nb);
   radix_scan_digits<<<dim3(R), dim3(SORT_THREADS), 0, stream>>>(block_hist, nb, digit_total);
   if (src_v2)
-    radix_scatter<2, KPT, R><<<grid, dim3(SORT_THREADS), 0, stream>>>(src_k, src_v, src_v2, dk, dv, dv2, n, n_dev,
-                                                                       shift, bits, block_hist, nb, digit_total);
+    radix_scatter<2, K, R, TH><<<grid, block, 0, stream>>>(src_k, src_v, src_v2, dk, dv, dv2, n, n_dev, shift, bits,
+                                                                  block_hist, nb, digit_total);
   else
-    radix_scatter<1, KPT, R><<<grid, dim3(SORT_THREADS), 0, stream>>>(src_k, src_v, nullptr, dk, dv, nullptr, n,
-                                                                       n_dev, shift, bits, block_hist, nb, digit_total);
+    radix_scatter<1, K, R, TH><<<grid, block, 0, stream>>>(src_k, src_v, nullptr, dk, dv, nullptr, n, n_dev, shift,
+                                                                  bits, block_hist, nb, digit_total);
 }
 
 }  // namespace
@@ -636,6 +737,10 @@ extern "C" int b2c_hip_radix_sort_kv2(const uint32_t* keys_in, const uint32_t* v
   const int kpt = sort_kpt(n);
   uint32_t* block_hist = static_cast<uint32_t*>(temp);
   uint32_t* digit_total = block_hist + (size_t)sort_blocks(n, kpt) * (kpt != KPT_SMALL ? 2 * RADIX : RADIX);
+  if (!two && !n_dev && n <= ONE_SORT_MAX) {
+    sort_one_kernel<<<1, ONE_THREADS, 0, stream>>>(keys_in, vals_in, keys_out, vals_out, n, begin_bit, end_bit);
+    return (int)hipGetLastError();
+  }
   // 8-bit digits; a large sort whose key width is a few bits over a multiple of 8 (17-bit tile keys at 4K)
   // widens the first passes to 9 bits instead of running a pass for the remainder
   const int width = end_bit - begin_bit;
@@ -659,21 +764,10 @@ extern "C" int b2c_hip_radix_sort_kv2(const uint32_t* keys_in, const uint32_t* v
     uint32_t* dk = to_out ? keys_out : keys_alt;
     uint32_t* dv = to_out ? vals_out : vals_alt;
     uint32_t* dv2 = two ? (to_out ? vals2_out : vals2_alt) : nullptr;
-    if (kpt == KPT_HUGE && bits > 8)
-      sort_pass<KPT_HUGE, 2 * RADIX>(src_k, src_v, src_v2, dk, dv, dv2, n, n_dev, shift, bits, block_hist, digit_total,
-                                     stream);
-    else if (kpt == KPT_HUGE)
-      sort_pass<KPT_HUGE, RADIX>(src_k, src_v, src_v2, dk, dv, dv2, n, n_dev, shift, bits, block_hist, digit_total,
-                                 stream);
-    else if (kpt == KPT_BIG && bits > 8)
-      sort_pass<KPT_BIG, 2 * RADIX>(src_k, src_v, src_v2, dk, dv, dv2, n, n_dev, shift, bits, block_hist, digit_total,
-                                    stream);
-    else if (kpt == KPT_BIG)
-      sort_pass<KPT_BIG, RADIX>(src_k, src_v, src_v2, dk, dv, dv2, n, n_dev, shift, bits, block_hist, digit_total,
-                                stream);
-    else
-      sort_pass<KPT_SMALL, RADIX>(src_k, src_v, src_v2, dk, dv, dv2, n, n_dev, shift, bits, block_hist, digit_total,
-                                  stream);
+    const auto pass = kpt == KPT_HUGE  ? (bits > 8 ? sort_pass<KPT_HUGE, 2 * RADIX> : sort_pass<KPT_HUGE, RADIX>)
+                      : kpt == KPT_BIG ? (bits > 8 ? sort_pass<KPT_BIG, 2 * RADIX> : sort_pass<KPT_BIG, RADIX>)
+                                       : sort_pass<KPT_SMALL, RADIX>;
+    pass(src_k, src_v, src_v2, dk, dv, dv2, n, n_dev, shift, bits, block_hist, digit_total, stream);
     int e = (int)hipGetLastError();
     if (e) return e;
     shift += bits;
@@ -712,7 +806,8 @@ extern "C" int b2c_hip_scan_counts_host(int n, const uint32_t* order, const uint
   if (temp_bytes < b2c_scan_temp_bytes((uint32_t)n)) return (int)hipErrorInvalidValue;
   const uint32_t nb = scan_blocks((uint32_t)n);
   uint32_t* block_sums = static_cast<uint32_t*>(temp);
-  scan_reduce<<<dim3(nb), dim3(SORT_THREADS), 0, stream>>>(n, order, tile_count, block_sums);
+  if (nb > 1)  // a single workgroup has no predecessors to sum
+    scan_reduce<<<dim3(nb), dim3(SORT_THREADS), 0, stream>>>(n, order, tile_count, block_sums);
   scan_down<<<dim3(nb), dim3(SORT_THREADS), 0, stream>>>(n, order, tile_count, block_sums, tile_off, total_dev,
                                                           total_host);
   return (int)hipGetLastError();
