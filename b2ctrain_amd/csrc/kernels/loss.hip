@@ -12,6 +12,7 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <algorithm>
 #include <mutex>
 
 namespace b2c {
@@ -41,7 +42,7 @@ __device__ __forceinline__ float gt_effective(uint32_t gp, int c, bool composite
 // steps past the strip's last row). Taller strips repeat fewer halo rows but make fewer, longer waves; the
 // launcher picks SH per image size and device (see pick_strip_rows).
 constexpr int SW = 54;
-constexpr int SH_MIN = 35, SH_MAX = 128;
+constexpr int SH_MIN = 35, SH_MAX = 128;  // (small images take shorter ones, see pick_strip_rows)
 
 struct PixelIn {
   float p, g;
@@ -365,22 +366,29 @@ LossSlots loss_slots() {
 }
 
 // Strip height. Every wave walks SH + 20 rows rounded up to whole rings, so the kernel takes about (rounds
-// of resident waves) x (rows walked); pick the height in [SH_MIN, SH_MAX] that minimises it for this image
+// of resident waves) x (rows walked); pick the height that minimises it for this image
 // and device, the tallest on ties (fewer waves). The kernel is VALU-bound: at 1080p heights 39 and 46 (one
 // round, 66 rows walked) measured the same, 94.6 and 94.2 us, and 60 (under two waves per SIMD) 96.4 us.
-// B2C_LOSS_STRIP_ROWS (a height in that range) overrides the choice, for tests and tuning.
+// Heights below SH_MIN walk mostly halo. They are taken only while every wave has a SIMD to itself (SHORT_WAVES at
+// most): its rows then cost their LDS latency, 0.95 us each, and 55.5 us became 20.9 us at 64x64 (22 rows for 66).
+// With two or three short waves a SIMD (800x800: 49.8 us against 64 us) the extra rows cost more than they give as
+// soon as other streams share the chip (training step 241 against 230 us with three in flight).
+// B2C_LOSS_STRIP_ROWS (a height from SH_MIN to SH_MAX) overrides the choice, for tests and tuning.
+constexpr long SHORT_WAVES = 1024;
+
 int pick_strip_rows(int W, int H) {
   if (const char* env = getenv("B2C_LOSS_STRIP_ROWS")) {
     const int v = atoi(env);
     if (v >= SH_MIN && v <= SH_MAX) return v;
   }
   const LossSlots sl = loss_slots();
-  const long slots = (long)sl.simds * sl.per_simd;
+  const long slots = (long)sl.simds * sl.per_simd, short_waves = std::min(SHORT_WAVES, (long)sl.simds);
   const int strips_x = (W + SW - 1) / SW;
   int best = SH_MIN;
   long best_cost = -1;
-  for (int sh = SH_MIN; sh <= SH_MAX; sh++) {
+  for (int sh = 1; sh <= SH_MAX; sh++) {
     const long waves = (long)strips_x * ((H + sh - 1) / sh) * 3;
+    if (sh < SH_MIN && waves > short_waves) continue;
     const long cost = ((waves + slots - 1) / slots) * ((sh + 4 * HALO + 10) / 11 * 11);
     if (best_cost < 0 || cost <= best_cost) {
       best_cost = cost;
@@ -474,7 +482,8 @@ extern "C" int b2c_hip_step_loss_sums(float* loss_accum, hipStream_t stream) {
 }
 
 extern "C" size_t b2c_loss_partials(int W, int H) {
-  return (size_t)((W + SW - 1) / SW) * ((H + SH_MIN - 1) / SH_MIN) * 3;  // the most strips any choice makes
+  // the most strips any choice makes
+  return std::max((size_t)((W + SW - 1) / SW) * ((H + SH_MIN - 1) / SH_MIN) * 3, (size_t)SHORT_WAVES);
 }
 
 extern "C" int b2c_hip_accumulate_loss(float* loss_accum, hipStream_t stream) {
