@@ -13,7 +13,7 @@ namespace {
 
 // Lanes are grouped by quadrant: lane 16 q + p is pixel p (row-major 4x4) of quadrant q (2x2 over the
 // tile). Each batch of up to 64 splats is staged in LDS together with one list per quadrant of the splats
-// whose ellipse can reach it (quadrant_mask), in depth order; the wave then runs max over quadrants of the
+// whose ellipse can reach it (quadrant_reach), in depth order; the wave then runs max over quadrants of the
 // list lengths iterations, each lane group taking the next splat of its own quadrant's list. A splat that
 // reaches no pixel of a quadrant would contribute alpha = 0 there, so the result equals the plain sweep.
 // The loop is branch-free: a lane that has terminated, has run out of its list, or whose fragment fails
@@ -95,7 +95,8 @@ __global__ void __launch_bounds__(64) raster_fwd_kernel(b2c_raster_fwd_args a) {
     if (ballot64(live) == 0) break;
     const uint32_t remaining = min(64u, range.y - start);
     __syncthreads();
-    uint32_t qmask = 0, gid = 0, gslot = 0;
+    Quadrants reach{};
+    uint32_t gid = 0, gslot = 0;
     if ((uint32_t)lane < remaining) {
       gid = a.vals_sorted[start + lane];
       if constexpr (COMPACT) gslot = a.slot_sorted[start + lane];
@@ -106,21 +107,9 @@ __global__ void __launch_bounds__(64) raster_fwd_kernel(b2c_raster_fwd_args a) {
       s_g1[lane] = make_float4(r0.w, r2.w, 0.f, r1.x);
       s_col[lane] = make_float4(r2.x, r2.y, r2.z, r1.z);
       if constexpr (EXT) s_ext[lane] = rec[3];
-      qmask = quadrant_mask(r0.x, r0.y, r0.z, r0.w, r1.x, r1.z, x0, y0);
+      reach = quadrant_reach(r0.x, r0.y, r0.z, r0.w, r1.x, r1.z, x0, y0);
     }
-    // per-quadrant lists: the lanes with bit qq set, in lane (depth) order, padded with the null splat
-    uint32_t n_iter = 0;
-    const uint64_t below = (1ull << lane) - 1ull;
-#pragma unroll
-    for (int qq = 0; qq < 4; qq++) {
-      const bool mine = (qmask >> qq) & 1u;
-      const uint64_t bal = ballot64(mine);
-      const uint32_t c = popc64(bal);
-      if (mine) s_list[qq][popc64(bal & below)] = (uint32_t)lane * 16u;
-      if ((uint32_t)lane >= c) s_list[qq][lane] = 64u * 16u;
-      n_iter = max(n_iter, c);
-    }
-    n_iter = __builtin_amdgcn_readfirstlane(n_iter);
+    const uint32_t n_iter = quadrant_lists(reach, lane, s_list);
     __syncthreads();
     const uint32_t* my_list = s_list[q];
     // The lists are walked in pairs (an odd count runs one null entry more); each offset register is
@@ -203,7 +192,7 @@ __global__ void __launch_bounds__(64) raster_fwd_kernel(b2c_raster_fwd_args a) {
       s_flag[lane] = 0u;  // cleared for the next batch (its flags are written after its lists are built)
       const uint64_t keep = ballot64(kept);
       if (kept) {
-        const uint32_t c = range.x + cbase + popc64(keep & below);
+        const uint32_t c = range.x + cbase + lanes_before(keep);
         a.cvals[c] = gid;
         a.cslots[c] = gslot;
       }

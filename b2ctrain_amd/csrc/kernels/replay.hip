@@ -335,7 +335,7 @@ __global__ void __launch_bounds__(64) probe_kernel(b2c_probe_args a) {
     if (ballot64(live) == 0ull) break;
     const uint32_t remaining = min(64u, range.y - start);
     __syncthreads();
-    uint32_t qmask = 0;
+    Quadrants reach{};
     if ((uint32_t)lane < remaining) {
       const uint32_t gid = a.vals_sorted[start + lane];
       const float4* rec = reinterpret_cast<const float4*>(a.raster_rec) + (size_t)gid * 4;
@@ -344,20 +344,9 @@ __global__ void __launch_bounds__(64) probe_kernel(b2c_probe_args a) {
       s_g0[lane] = make_float4(def.x, def.y, def.z, r0.z);
       s_g1[lane] = make_float4(r0.w, r2.w, r1.z, r1.x);  // (c01, log2 opacity, power, c11 / 2)
       s_z[lane] = r3.w;
-      qmask = quadrant_mask(r0.x, r0.y, r0.z, r0.w, r1.x, r1.z, x0, y0);
+      reach = quadrant_reach(r0.x, r0.y, r0.z, r0.w, r1.x, r1.z, x0, y0);
     }
-    uint32_t n_iter = 0;
-    const uint64_t below = (1ull << lane) - 1ull;
-#pragma unroll
-    for (int qq = 0; qq < 4; qq++) {
-      const bool mine = (qmask >> qq) & 1u;
-      const uint64_t bal = ballot64(mine);
-      const uint32_t c = popc64(bal);
-      if (mine) s_list[qq][popc64(bal & below)] = (uint32_t)lane * 16u;
-      if ((uint32_t)lane >= c) s_list[qq][lane] = 64u * 16u;
-      n_iter = max(n_iter, c);
-    }
-    n_iter = __builtin_amdgcn_readfirstlane(n_iter);
+    const uint32_t n_iter = quadrant_lists(reach, lane, s_list);
     __syncthreads();
     const uint32_t* my_list = s_list[q];
     uint32_t off0 = my_list[0], off1 = my_list[1];

@@ -1,5 +1,5 @@
-"""The forward raster's quadrant culling test (quadrant_mask in b2ctrain_amd/csrc/kernels/raster_common.h),
-restated in float32 numpy, must be conservative: a quadrant with a pixel centre where the raster kernels'
+"""The raster's quadrant culling test by the edges of each quadrant (which quadrant_reach in
+b2ctrain_amd/csrc/kernels/raster_common.h evaluates by lines, see test_quadrant_reach.py), in float32 numpy, must be conservative: a quadrant with a pixel centre where the raster kernels'
 fp32 sigma (the quadratic about the tile centre of sigma_coefs / poly_sigma, five fused multiply-adds,
 evaluated here by the oracle's C restatement; the reference's src/gpu/raster_fwd.cu:44-50 rounds the same
 quantity differently) passes sigma <= power must keep its bit. Checked by brute force over all 64 pixel centres on random splats,
@@ -23,7 +23,7 @@ def edge_lb(ah, b, ch, dx, dy):
 
 def poly_slack_power(mx, my, ah, b, ch, power, x0, y0):
     """power raised by 1e-5 of the magnitude of the tile-centred quadratic's terms over the tile (the
-    per-pixel sigma's rounding scale), as quadrant_mask does."""
+    per-pixel sigma's rounding scale), as the kernels do."""
     mxr, myr, bb = np.abs(mx - (x0 + f32(3.5))), np.abs(my - (y0 + f32(3.5))), np.abs(b)
     scale = (((ah * mxr + bb * myr) * mxr + ch * myr * myr) +
              f32(3.5) * ((f32(2) * ah + bb) * mxr + (bb + f32(2) * ch) * myr) + f32(12.25) * (ah + bb + ch))
@@ -31,7 +31,7 @@ def poly_slack_power(mx, my, ah, b, ch, power, x0, y0):
 
 
 def quadrant_mask(mx, my, ah, b, ch, power, x0, y0):
-    """Restates raster_common.h's quadrant_mask: per quadrant, the centre inside the box, or the clamped
+    """Per quadrant, the centre inside the box, or the clamped
     minimum on the (at most one) vertical and (at most one) horizontal edge the centre lies beyond."""
     with np.errstate(all="ignore"):
         power = poly_slack_power(mx, my, ah, b, ch, power, x0, y0)
