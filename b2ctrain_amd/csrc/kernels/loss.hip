@@ -386,10 +386,13 @@ int pick_strip_rows(int W, int H) {
   const int strips_x = (W + SW - 1) / SW;
   int best = SH_MIN;
   long best_cost = -1;
-  for (int sh = 1; sh <= SH_MAX; sh++) {
+  // of the heights that walk the same rings the tallest has the fewest waves, so only those are weighed (every height in
+  // turn cost the launch ten times the divisions)
+  for (int rings = 2; 11 * (rings - 1) < SH_MAX + 4 * HALO; rings++) {
+    const int sh = std::min(11 * rings - 4 * HALO, SH_MAX);
     const long waves = (long)strips_x * ((H + sh - 1) / sh) * 3;
     if (sh < SH_MIN && waves > short_waves) continue;
-    const long cost = ((waves + slots - 1) / slots) * ((sh + 4 * HALO + 10) / 11 * 11);
+    const long cost = ((waves + slots - 1) / slots) * (11 * rings);
     if (best_cost < 0 || cost <= best_cost) {
       best_cost = cost;
       best = sh;
