@@ -34,6 +34,10 @@ constexpr uint32_t BIG_SORT_MIN = 1u << 22;
 constexpr int KPT_BIG = 16;    // 4096-key tiles
 constexpr int KPT_HUGE = 32;   // 8192-key tiles, from HUGE_SORT_MIN keys
 constexpr uint32_t HUGE_SORT_MIN = 1u << 25;
+// Up to FUSE_TILES tiles (131072 keys, their number known to the host) the histograms stay raw and by tile, and each
+// scatter workgroup sums the tiles before its own itself, coalesced, instead of the digit scan's launch between: 131.6 ->
+// 125.5 us of binning at 49 tiles, the same time at 74 and 98 tiles (and a launch less), 141 -> 146 us at 123 and 163.
+constexpr uint32_t FUSE_TILES = 64;
 // Sorts of up to ONE_SORT_MAX keys (their number known to the host, one value array) run in one workgroup.
 constexpr int ONE_THREADS = 1024, ONE_KPT = 4;
 constexpr uint32_t ONE_SORT_MAX = ONE_THREADS * ONE_KPT;
@@ -105,8 +109,9 @@ __device__ __forceinline__ uint32_t sort_tile(uint32_t nblocks) {
 // Per-tile digit histogram (R = 256 or 512 digits). Thread t loads the KPT consecutive keys [t KPT, t KPT +
 // KPT) of the tile (16-byte loads) and counts runs of one digit in registers, adding each run to the LDS
 // histogram with one atomic: tile keys in emit order come in runs (a splat's tiles along a bbox row), which
-// would otherwise serialise on the same LDS word.
-template <int KPT, int R>
+// would otherwise serialise on the same LDS word. The counts go out digit by digit (a row of tiles each, for the digit
+// scan), or BY_TILE.
+template <int KPT, int R, bool BY_TILE>
 __global__ void __launch_bounds__(SORT_THREADS) radix_upsweep(const uint32_t* __restrict__ keys, uint32_t cap,
                                                               const uint32_t* __restrict__ n_dev, int shift, int bits,
                                                               uint32_t* __restrict__ block_hist, uint32_t nblocks) {
@@ -149,7 +154,7 @@ __global__ void __launch_bounds__(SORT_THREADS) radix_upsweep(const uint32_t* __
     if (run_c) atomicAdd(&hist[run_d], run_c);
   }
   __syncthreads();
-  for (int t = threadIdx.x; t < R; t += SORT_THREADS) block_hist[(size_t)t * nblocks + tile] = hist[t];
+  for (int t = threadIdx.x; t < R; t += SORT_THREADS) block_hist[BY_TILE ? (size_t)tile * R + t : (size_t)t * nblocks + tile] = hist[t];
 }
 
 // One workgroup per digit: exclusive scan of the digit's per-tile counts (each thread a contiguous run of
@@ -196,7 +201,7 @@ __global__ void __launch_bounds__(SORT_THREADS) radix_scan_digits(uint32_t* __re
 // staging buffer sorted by digit, which is written out in order: each digit's keys of this tile form one
 // contiguous run in the output, so consecutive lanes write consecutive addresses. NV = 1 or 2 value arrays
 // ride along with the keys. R = 256 or 512 digits (8- or 9-bit passes); thread t owns digits t R/256 ...
-template <int NV, int KPT, int R, int TH>
+template <int NV, int KPT, int R, int TH, bool FUSED>
 __global__ void __launch_bounds__(TH) radix_scatter(
     const uint32_t* __restrict__ keys_in, const uint32_t* __restrict__ vals_in, const uint32_t* __restrict__ vals2_in,
     uint32_t* __restrict__ keys_out, uint32_t* __restrict__ vals_out, uint32_t* __restrict__ vals2_out, uint32_t cap,
@@ -234,8 +239,32 @@ __global__ void __launch_bounds__(TH) radix_scatter(
   uint32_t loff_d[DPT];  // local (staging) offset of each of this thread's digits
   {  // 2. thread t owns digits t DPT .. t DPT + DPT - 1: global base and local offset of each in this tile
     uint32_t tot_d[DPT], mine[DPT], cnt[DPT], tot_sum = 0, cnt_sum = 0;
+    if constexpr (FUSED) {  // raw counts by tile: thread d and thread R + d each sum half of the tiles, 1 KB a tile
+      static_assert(TH == 2 * R && DPT == 1 && TILE >= 3 * R, "two threads per digit; the sums meet in s_key");
+      const uint32_t d = threadIdx.x & (R - 1), half = (nblocks + 1u) / 2u;
+      const uint32_t lo = threadIdx.x < R ? 0u : half, hi = threadIdx.x < R ? half : nblocks;
+      uint32_t all = 0u, before = 0u, here = 0u;
+#pragma unroll 8
+      for (uint32_t t = lo; t < hi; t++) {
+        const uint32_t c = block_hist[(size_t)t * R + d];
+        all += c;
+        before += t < tile ? c : 0u;
+        here += t == tile ? c : 0u;
+      }
+      if (threadIdx.x >= R) {
+        s_key[d] = all;
+        s_key[R + d] = before;
+        s_key[2 * R + d] = here;
+      }
+      __syncthreads();
+      tot_d[0] = has_digits ? all + s_key[d] : 0u;
+      mine[0] = has_digits ? before + s_key[R + d] : 0u;
+      cnt[0] = has_digits ? here + s_key[2 * R + d] : 0u;
+      tot_sum = tot_d[0];
+      cnt_sum = cnt[0];
+    }
 #pragma unroll
-    for (int j = 0; j < DPT; j++) {
+    for (int j = 0; j < (FUSED ? 0 : DPT); j++) {
       const uint32_t d = has_digits ? threadIdx.x * DPT + j : 0u;
       tot_d[j] = has_digits ? digit_total[d] : 0u;
       mine[j] = has_digits ? block_hist[(size_t)d * nblocks + tile] : 0u;
@@ -699,13 +728,25 @@ void sort_pass(const uint32_t* src_k, const uint32_t* src_v, const uint32_t* src
   const dim3 grid(8u * ((nb + 7u) / 8u));  // sort_tile's XCD-contiguous mapping
   constexpr int TH = SCATTER_THREADS, K = KPT * SORT_THREADS / TH;
   const dim3 block(TH);
-  radix_upsweep<KPT, R><<<grid, dim3(SORT_THREADS), 0, stream>>>(src_k, n, n_dev, shift, bits, block_hist, nb);
+  if constexpr (KPT == KPT_SMALL && R == RADIX) {
+    if (nb <= FUSE_TILES && !n_dev) {
+      radix_upsweep<KPT, R, true><<<grid, dim3(SORT_THREADS), 0, stream>>>(src_k, n, n_dev, shift, bits, block_hist, nb);
+      if (src_v2)
+        radix_scatter<2, K, R, TH, true><<<grid, block, 0, stream>>>(src_k, src_v, src_v2, dk, dv, dv2, n, n_dev, shift,
+                                                                     bits, block_hist, nb, digit_total);
+      else
+        radix_scatter<1, K, R, TH, true><<<grid, block, 0, stream>>>(src_k, src_v, nullptr, dk, dv, nullptr, n, n_dev,
+                                                                     shift, bits, block_hist, nb, digit_total);
+      return;
+    }
+  }
+  radix_upsweep<KPT, R, false><<<grid, dim3(SORT_THREADS), 0, stream>>>(src_k, n, n_dev, shift, bits, block_hist, nb);
   radix_scan_digits<<<dim3(R), dim3(SORT_THREADS), 0, stream>>>(block_hist, nb, digit_total);
   if (src_v2)
-    radix_scatter<2, K, R, TH><<<grid, block, 0, stream>>>(src_k, src_v, src_v2, dk, dv, dv2, n, n_dev, shift, bits,
+    radix_scatter<2, K, R, TH, false><<<grid, block, 0, stream>>>(src_k, src_v, src_v2, dk, dv, dv2, n, n_dev, shift, bits,
                                                                   block_hist, nb, digit_total);
   else
-    radix_scatter<1, K, R, TH><<<grid, block, 0, stream>>>(src_k, src_v, nullptr, dk, dv, nullptr, n, n_dev, shift,
+    radix_scatter<1, K, R, TH, false><<<grid, block, 0, stream>>>(src_k, src_v, nullptr, dk, dv, nullptr, n, n_dev, shift,
                                                                   bits, block_hist, nb, digit_total);
 }
 

@@ -1,4 +1,5 @@
-"""The one-workgroup sort (up to 4096 keys, csrc/kernels/binning.hip) at the edges of its waves and rounds, against
+"""The small sorts of csrc/kernels/binning.hip: one workgroup (up to 4096 keys) at the edges of its waves and rounds, and up to
+64 tiles without a digit scan, against
 numpy's stable argsort; the same keys with a second value array take the general passes and must agree too."""
 import numpy as np
 import pytest
@@ -27,3 +28,15 @@ def test_one_workgroup_sort(n, begin, end, keys):
     ko, vo, v2o = _sort(k, v, v2, begin, end)
     ek, ev, ev2 = _expect(k, v, v2, begin, end)
     assert np.array_equal(ko, ek) and np.array_equal(vo, ev) and np.array_equal(v2o, ev2)
+
+
+@pytest.mark.parametrize("n", [4097, 6144, 6145, 131_071, 131_072, 131_073])
+@pytest.mark.parametrize("begin,end,two", [(0, 32, False), (5, 18, True), (0, 8, False)])
+def test_scatter_sums_the_tiles_before_it(n, begin, end, two):
+    """Sorts of up to 64 tiles of 2048 keys have no digit scan; one key more has."""
+    rng = np.random.default_rng(n + end)
+    k, v, v2 = (rng.integers(0, 2 ** 32, n, dtype=np.uint64).astype(np.uint32) for _ in range(3))
+    k[rng.random(n) < 0.3] = 0xFFFFFFFF
+    got, want = _sort(k, v, v2 if two else None, begin, end), _expect(k, v, v2 if two else None, begin, end)
+    for g, w in zip(got, want):
+        assert (g is None and w is None) or np.array_equal(g, w)
