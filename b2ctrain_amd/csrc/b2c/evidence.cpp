@@ -11,8 +11,9 @@ namespace {
 DevBuf<float> g_evidence;  // [n][B2C_EVIDENCE_STRIDE]
 DevBuf<float> g_view_acc;  // [n][3] the current view's (w_in, err, w_all)
 DevBuf<float> g_labels;    // [n][B2C_LABEL_BINS]
-// The downloads' rows, formed on the device from the accumulators (sized with them; every download of one
-// pass writes the same values).
+// The downloads' rows, formed on the device from the accumulators (every download of one pass writes the same
+// values). They are reserved before their accumulators, so an accumulator that holds n splats has n rows beside it
+// also after a reserve has thrown.
 DevBuf<float> g_evidence_rows;  // [n][7]
 DevBuf<float> g_label_rows;     // [n][2]
 bool g_labels_valid = false;
@@ -22,15 +23,15 @@ void compute_evidence(RenderCtx& ctx, const Model& m, const std::vector<ViewGPU>
                       const EvidenceParams& cfg, hipStream_t stream) {
   if (views.size() != cams.size()) throw std::runtime_error("compute_evidence: one camera per view");
   const size_t n = (size_t)(m.n > 0 ? m.n : 1);
+  g_evidence_rows.reserve(n * 7);
   g_evidence.reserve(n * B2C_EVIDENCE_STRIDE);
   g_evidence.zero(stream);
-  g_evidence_rows.reserve(n * 7);
   g_view_acc.reserve(n * 3);
   g_labels_valid = cfg.export_labels;
   if (g_labels_valid) {
+    g_label_rows.reserve(n * 2);
     g_labels.reserve(n * B2C_LABEL_BINS);
     g_labels.zero(stream);
-    g_label_rows.reserve(n * 2);
   }
   const bool use_normals = cfg.evidence_normal_weight > 0.f;
   for (size_t v = 0; v < views.size(); v++) {
