@@ -124,7 +124,8 @@ __device__ __forceinline__ int anchor_value(int lane) {
 
 // T / keep and Q / keep for keep in [0.001, 0.997]: one reciprocal refined by a Newton step, then each quotient
 // corrected by its own remainder (the steps of an IEEE division without the scaling that keep's range does not
-// need): 9 operations instead of two divisions' 24.
+// need): 10 operations instead of two divisions' 24. T is a transmittance in [0, 1]; Q is any float, and the remainder of
+// an infinite quotient, itself infinite or NaN, is made finite so that the quotient stays infinite.
 struct Quotients {
   float t, q;
 };
@@ -132,7 +133,8 @@ __device__ __forceinline__ Quotients divide_both(float t, float q, float keep) {
   float r = __builtin_amdgcn_rcpf(keep);
   r = __builtin_fmaf(__builtin_fmaf(-keep, r, 1.f), r, r);
   const float t0 = t * r, q0 = q * r;
-  return Quotients{__builtin_fmaf(__builtin_fmaf(-keep, t0, t), r, t0), __builtin_fmaf(__builtin_fmaf(-keep, q0, q), r, q0)};
+  const float q_rem = __builtin_amdgcn_fmed3f(__builtin_fmaf(-keep, q0, q), -__FLT_MAX__, __FLT_MAX__);
+  return Quotients{__builtin_fmaf(__builtin_fmaf(-keep, t0, t), r, t0), __builtin_fmaf(q_rem, r, q0)};
 }
 
 template <bool FEAT, bool HOLLOW>
