@@ -45,8 +45,6 @@ __global__ void __launch_bounds__(64) evidence_kernel(b2c_evidence_args a) {
   __shared__ uint32_t s_id[64];
   __shared__ __attribute__((aligned(16))) float s_vis[EG * VSTRIDE];
   __shared__ __attribute__((aligned(16))) float s_kc[LABELS ? MAXC : 1][64];  // k of the tile's c-th class's pixels, else 0
-  __shared__ uint32_t s_lab[64];                 // class of the pixels beyond the first MAXC classes
-  __shared__ float s_kv[LABELS ? 64 : 1];
   __shared__ uint32_t s_slot[64];
   const TileAt here = xcd_tile(blockIdx.x, a.tiles_x, a.tiles_y);
   const int tile = here.tile;
@@ -99,7 +97,6 @@ __global__ void __launch_bounds__(64) evidence_kernel(b2c_evidence_args a) {
   s_vis[lane] = m;
   s_vis[64 + lane] = mres;
   s_vis[128 + lane] = k;
-  if constexpr (LABELS) s_kv[lane] = k;
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < 16; i++) {
@@ -109,7 +106,8 @@ __global__ void __launch_bounds__(64) evidence_kernel(b2c_evidence_args a) {
   }
   uint32_t cls[MAXC] = {0u, 0u, 0u, 0u};  // wave-uniform: the tile's first classes, in pixel order
   int ncls = 0;
-  bool rest = false;  // a pixel's class is not among them
+  uint32_t rest = 0;  // the classes past those, one bit each
+  uint32_t pl[4] = {};  // and this lane's quarter of the pixels' class among them, a byte each (LABEL_BINS: none)
   if constexpr (LABELS) {
     uint64_t todo = ballot64(lab != LABEL_NONE);
     int my_c = -1;
@@ -120,10 +118,21 @@ __global__ void __launch_bounds__(64) evidence_kernel(b2c_evidence_args a) {
       cls[ncls++] = b;
       todo &= ~hit;
     }
-    rest = todo != 0ull;
 #pragma unroll
     for (int c = 0; c < MAXC; c++) s_kc[c][lane] = my_c == c ? k : 0.f;
-    s_lab[lane] = my_c < 0 ? lab : LABEL_NONE;
+    const uint32_t mine = my_c < 0 ? min(lab, (uint32_t)B2C_LABEL_BINS) : (uint32_t)B2C_LABEL_BINS;
+    while (todo != 0ull) {
+      const uint32_t b = (uint32_t)__builtin_amdgcn_readlane((int)mine, __builtin_ctzll(todo));
+      rest |= 1u << b;
+      todo &= ~ballot64(mine == b);
+    }
+    if (rest != 0u) {
+      __syncthreads();  // the pixel vectors are read
+      reinterpret_cast<uint8_t*>(s_vis)[lane] = (uint8_t)mine;
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < 4; i++) pl[i] = reinterpret_cast<const uint32_t*>(s_vis)[eq * 4 + i];
+    }
   }
   float T = 1.f;
   for (uint32_t start = range.x; start < range.y; start += 64) {
@@ -190,24 +199,13 @@ __global__ void __launch_bounds__(64) evidence_kernel(b2c_evidence_args a) {
           sum = sum_quarters(sum);
           if (eq == 0 && e < count && sum != 0.f) atomicAdd(bins + cls[c], sum);
         }
-        if (rest && eq == 0 && e < count) {  // classes past the first MAXC of the tile: one pass each
-          uint64_t todo = ~0ull;
-          while (true) {
-            uint32_t b = LABEL_NONE;
-            for (int p = 0; p < 64; p++)
-              if (((todo >> p) & 1ull) && s_lab[p] != LABEL_NONE) {
-                b = s_lab[p];
-                break;
-              }
-            if (b == LABEL_NONE) break;
-            float sum = 0.f;
-            for (int p = 0; p < 64; p++)
-              if (s_lab[p] == b) {
-                sum += row[p] * s_kv[p];
-                todo &= ~(1ull << p);
-              }
-            if (sum != 0.f) atomicAdd(bins + b, sum);
-          }
+        for (uint32_t left = rest; left != 0u; left &= left - 1u) {  // wave-uniform
+          const uint32_t b = (uint32_t)__builtin_ctz(left);
+          float sum = 0.f;
+#pragma unroll
+          for (int i = 0; i < 16; i++) sum += ((pl[i / 4] >> (8 * (i % 4))) & 0xFFu) == b ? row[eq * 16 + i] * pk[i] : 0.f;
+          sum = sum_quarters(sum);
+          if (eq == 0 && e < count && sum != 0.f) atomicAdd(bins + b, sum);
         }
       }
       __syncthreads();  // the group's rows are consumed
