@@ -28,7 +28,10 @@ __device__ __forceinline__ float byte_chan(uint32_t p, int c) { return (float)((
 // LABELS the tile's distinct classes are found once (ballots: labels are spatially coherent, a tile usually
 // holds one or two), each with a pixel vector k * [pixel in the class]; the same rows are contracted with
 // those vectors and added to the splat's class bins with float atomics. Classes beyond the first MAXC of a
-// tile take a slower pass over the pixels. With all 64 splats of a batch in the matrix (17 KB) a CU held 9 waves, and every
+// tile take a sum masked by class each, over the same quarters (the classes of a lane's quarter of the pixels are four
+// registers of bytes): a pass with labels over 200k splats at 800x800 takes 622 us with classes of 5x5 pixels and 1916 us
+// with a class for every pixel, against 1206 and 5187 us where 16 lanes walk the pixels of a class one by one.
+// With all 64 splats of a batch in the matrix (17 KB) a CU held 9 waves, and every
 // lane read the three pixel vectors from LDS for each row: 125 -> 92 us a 960x720 view with labels.
 constexpr int EG = 16;   // splats per group
 constexpr int MAXC = 4;  // classes per tile with their own pixel vector
