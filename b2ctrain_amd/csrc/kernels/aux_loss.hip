@@ -19,7 +19,8 @@ constexpr int AUX_GRID_MAX = 2048;  // grid-stride kernels: at most this many wo
 
 // Sum of one value over a 256-thread workgroup: wave shuffles, then the four wave totals in LDS, added by
 // thread 0 in wave order.
-__device__ __forceinline__ float block_sum(float v, float* s_red) {
+template <typename T>
+__device__ __forceinline__ T block_sum(T v, T* s_red) {
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o);
   __syncthreads();  // s_red may still be read from a previous call
@@ -81,14 +82,89 @@ __global__ void __launch_bounds__(AUX_BLOCK) hollow_sum_kernel(const float* __re
 
 // Eval metrics (loss.cu:240-286): the prediction clamped to [0, 1] and rounded to 8 bits against the target, per channel
 // the squared error and the clamped SSIM (both weighted by the target alpha when mask_weighted; zero outside the
-// image). One wave per (strip, channel): a strip is EW = 54 output columns by `rows` output rows, lane l owns column
+// image), summed in double. Large images take eval_kernel, small ones eval_tile_kernel.
+constexpr int ESTATS = 5;  // E[x], E[x^2], E[y], E[y^2], E[xy]
+
+__device__ __forceinline__ float eval_pred(float p) { return __builtin_rintf(fminf(fmaxf(p, 0.f), 1.f) * 255.f) / 255.f; }
+
+// The blurred statistics of one row: 11 taps of (u, v), added to st.
+__device__ __forceinline__ void eval_tap(float w, float u, float v, float (&st)[ESTATS]) {
+  const float wu = w * u, wv = w * v;
+  st[0] = st[0] + wu;
+  st[1] = __builtin_fmaf(wu, u, st[1]);
+  st[2] = st[2] + wv;
+  st[3] = __builtin_fmaf(wv, v, st[3]);
+  st[4] = __builtin_fmaf(wu, v, st[4]);
+}
+
+__device__ __forceinline__ float eval_ssim(const float (&st)[ESTATS]) {
+  const float mu1 = st[0], mu2 = st[2];
+  const float s1 = fmaxf(0.f, st[1] - mu1 * mu1), s2 = fmaxf(0.f, st[3] - mu2 * mu2), s12 = st[4] - mu1 * mu2;
+  const float num = ((2.f * mu1) * mu2 + C1) * (2.f * s12 + C2);
+  const float den = ((mu1 * mu1 + mu2 * mu2) + C1) * ((s1 + s2) + C2);
+  return fminf(fmaxf(num / den, -1.f), 1.f);
+}
+
+// One 256-thread workgroup per 16x16 tile and channel: the 26x26 input footprint and the horizontally blurred
+// statistics of its rows in LDS, a thread per output pixel. A tile's chain is short (load, two blurs) where a strip
+// walks at least 33 rows of 0.6 us each, so it is the faster one while the tiles leave the chip room.
+constexpr int ET = 16;              // output tile edge
+constexpr int EIN = ET + 2 * HALO;  // 26: input footprint edge
+
+__global__ void __launch_bounds__(AUX_BLOCK) eval_tile_kernel(b2c_eval_args a, int tiles_x) {
+  __shared__ float s_p[EIN * EIN], s_g[EIN * EIN];
+  __shared__ float s_h[EIN * ET][ESTATS];
+  __shared__ double s_red[4];
+  const int c = blockIdx.y, x0 = ((int)blockIdx.x % tiles_x) * ET, y0 = ((int)blockIdx.x / tiles_x) * ET;
+  const int tid = threadIdx.x;
+  for (int i = tid; i < EIN * EIN; i += AUX_BLOCK) {
+    const int y = y0 - HALO + i / EIN, x = x0 - HALO + i % EIN;
+    const bool in = x >= 0 && x < a.W && y >= 0 && y < a.H;
+    const size_t pix = in ? (size_t)y * a.W + x : 0;
+    s_p[i] = in ? eval_pred(a.pred[pix * 4 + c]) : 0.f;
+    s_g[i] = in ? gt_channel(a.gt[pix], c) : 0.f;
+  }
+  __syncthreads();
+  for (int i = tid; i < EIN * ET; i += AUX_BLOCK) {
+    const int first = (i / ET) * EIN + i % ET;
+    float st[ESTATS] = {0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int d = 0; d < 11; d++) eval_tap(gw_tap(d), s_p[first + d], s_g[first + d], st);
+#pragma unroll
+    for (int k = 0; k < ESTATS; k++) s_h[i][k] = st[k];
+  }
+  __syncthreads();
+  const int ly = tid / ET, lx = tid % ET, y = y0 + ly, x = x0 + lx;
+  double se = 0.0, ss = 0.0;
+  if (x < a.W && y < a.H) {
+    float st[ESTATS] = {0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int d = 0; d < 11; d++) {
+#pragma unroll
+      for (int k = 0; k < ESTATS; k++) st[k] = __builtin_fmaf(gw_tap(d), s_h[(ly + d) * ET + lx][k], st[k]);
+    }
+    const int i = (ly + HALO) * EIN + lx + HALO;
+    const float m = a.mask_weighted ? gt_channel(a.gt[(size_t)y * a.W + x], 3) : 1.f;
+    const float d = fabsf(s_p[i] - s_g[i]) * m;
+    se = (double)(d * d);
+    ss = (double)(eval_ssim(st) * m);
+  }
+  const double tse = block_sum(se, s_red);
+  const double tss = block_sum(ss, s_red);
+  if (tid == 0) {
+    const size_t wg = (size_t)blockIdx.y * gridDim.x + blockIdx.x;
+    a.partials[2 * wg] = (float)tse;
+    a.partials[2 * wg + 1] = (float)tss;
+  }
+}
+
+// One wave per (strip, channel): a strip is EW = 54 output columns by `rows` output rows, lane l owns column
 // x0 - 5 + l and walks down the rows. A step loads one row (a step ahead), blurs it horizontally through a one-row LDS
 // buffer into an 11-row register ring of the five statistics, and blurs the ring vertically; unrolled by 11, so the
 // ring slots are static registers. Each lane adds its rows' terms in double; the wave's two sums go to partials.
 // Bound by the VALU: 16x16 tiles with both passes in LDS re-read 2.6 times the pixels, ran 1.6 times the horizontal blurs,
 // kept the statistics in LDS and took 68.4 us at 1600x900; this takes 38.8 us.
 constexpr int EW = 64 - 2 * HALO;
-constexpr int ESTATS = 5;  // E[x], E[x^2], E[y], E[y^2], E[xy]
 
 __global__ void __launch_bounds__(64) eval_kernel(b2c_eval_args a, int strips_x, int nstrips, int rows) {
   __shared__ float s_p[2][64], s_g[2][64];  // one input row (double buffered)
@@ -118,7 +194,7 @@ __global__ void __launch_bounds__(64) eval_kernel(b2c_eval_args a, int strips_x,
       p_next = a.pred[pix * 4 + c];
       g_next = a.gt[pix];
       const bool in = col_in && y >= 0 && y < a.H;
-      const float p = in ? __builtin_rintf(fminf(fmaxf(p_raw, 0.f), 1.f) * 255.f) / 255.f : 0.f;
+      const float p = in ? eval_pred(p_raw) : 0.f;
       const float g = in ? gt_channel(g_raw, c) : 0.f;
       mm[j] = a.mask_weighted ? gt_channel(g_raw, 3) : 1.f;
       dm[j] = fabsf(p - g) * mm[j];
@@ -127,16 +203,7 @@ __global__ void __launch_bounds__(64) eval_kernel(b2c_eval_args a, int strips_x,
       __syncthreads();
       float st[ESTATS] = {0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int d = 0; d < 11; d++) {
-        const float w = gw_tap(d);
-        const float u = s_p[buf][first + d], v = s_g[buf][first + d];
-        const float wu = w * u, wv = w * v;
-        st[0] = st[0] + wu;
-        st[1] = __builtin_fmaf(wu, u, st[1]);
-        st[2] = st[2] + wv;
-        st[3] = __builtin_fmaf(wv, v, st[3]);
-        st[4] = __builtin_fmaf(wu, v, st[4]);
-      }
+      for (int d = 0; d < 11; d++) eval_tap(gw_tap(d), s_p[buf][first + d], s_g[buf][first + d], st);
 #pragma unroll
       for (int k = 0; k < ESTATS; k++) ring[j][k] = st[k];
       if (r < 2 * HALO) continue;
@@ -150,15 +217,10 @@ __global__ void __launch_bounds__(64) eval_kernel(b2c_eval_args a, int strips_x,
 #pragma unroll
         for (int k = 0; k < ESTATS; k++) st[k] = __builtin_fmaf(w, ring[(j + 1 + d) % 11][k], st[k]);  // oldest row first
       }
-      const float mu1 = st[0], mu2 = st[2];
-      const float s1 = fmaxf(0.f, st[1] - mu1 * mu1), s2 = fmaxf(0.f, st[3] - mu2 * mu2), s12 = st[4] - mu1 * mu2;
-      const float num = ((2.f * mu1) * mu2 + C1) * (2.f * s12 + C2);
-      const float den = ((mu1 * mu1 + mu2 * mu2) + C1) * ((s1 + s2) + C2);
-      const float ssim = fminf(fmaxf(num / den, -1.f), 1.f);
       const int slot = (j + 6) % 11;  // row yo
       if (out_lane) {
         se += (double)(dm[slot] * dm[slot]);
-        ss += (double)(ssim * mm[slot]);
+        ss += (double)(eval_ssim(st) * mm[slot]);
       }
     }
   }
@@ -173,16 +235,22 @@ __global__ void __launch_bounds__(64) eval_kernel(b2c_eval_args a, int strips_x,
   }
 }
 
+// The partials hold one entry per channel and tile.
+int eval_tiles(int W, int H) { return ((W + ET - 1) / ET) * ((H + ET - 1) / ET); }
+
 // Rows of a strip, so that with its halo it walks whole rings of 11: as few walked rows as possible
-// while at most two waves a SIMD run (a row then costs its latency), beyond that the least waves times rows. 23 rows at
-// least, so strips never outnumber the 16x16 tiles that size the partials.
+// while at most two waves a SIMD (2048 on the 1024 SIMDs) run, whose rows then cost their latency, beyond that the least
+// waves times rows. 23 rows at least, so strips never outnumber the 16x16 tiles that size the partials. 0: the tile
+// kernel, where a tile, as long as 50 of those waves times rows, makes it the faster one. Tiles against strips:
+// 7.1 and 21.3 us at 64x64, 13.3 and 21.8 us at 400x400, 20.7 and 22.0 us at 768x432 (1296 tiles); 23.6 and 22.1 us at
+// 640x640 (1600), 68.7 and 38.7 us at 1600x900; 27.3 and 36.5 us at 16x30000, whose strips are 16 of 54 columns wide.
 int eval_strip_rows(int W, int H) {
   const long strips_x = (W + EW - 1) / EW, resident = 2048;
-  int best = 23;
-  long best_cost = -1;
+  int best = 0;
+  long best_cost = 50L * eval_tiles(W, H);
   for (int rows = 23; rows <= 122; rows += 11) {
     const long cost = std::max(strips_x * ((H + rows - 1) / rows) * 3, resident) * (rows + 2 * HALO);
-    if (best_cost < 0 || cost < best_cost) {
+    if (cost < best_cost) {
       best_cost = cost;
       best = rows;
     }
@@ -227,9 +295,6 @@ int aux_grid(int npix) {
   return blocks < AUX_GRID_MAX ? blocks : AUX_GRID_MAX;
 }
 
-constexpr int ET = 16;  // the partials hold one entry per channel and 16x16 tile
-int eval_tiles(int W, int H) { return ((W + ET - 1) / ET) * ((H + ET - 1) / ET); }
-
 }  // namespace
 }  // namespace dev
 }  // namespace b2c
@@ -266,9 +331,15 @@ extern "C" int b2c_hip_hollow_loss(const float* hollow_pen, int W, int H, float 
 extern "C" int b2c_hip_eval_metrics(const b2c_eval_args* a, hipStream_t stream) {
   if (a->W <= 0 || a->H <= 0) return 0;
   if (!a->pred || !a->gt || !a->loss_accum || !a->partials) return (int)hipErrorInvalidValue;
-  const int strips_x = (a->W + EW - 1) / EW, rows = eval_strip_rows(a->W, a->H);
-  const int nstrips = strips_x * ((a->H + rows - 1) / rows);
-  eval_kernel<<<8 * ((nstrips * 3 + 7) / 8), 64, 0, stream>>>(*a, strips_x, nstrips, rows);
-  aux_reduce_kernel<<<1, 1024, 0, stream>>>(a->partials, nstrips * 3, 1, 1.f, a->loss_accum, 4);
+  const int rows = eval_strip_rows(a->W, a->H);
+  int count = eval_tiles(a->W, a->H) * 3;
+  if (rows == 0) {
+    eval_tile_kernel<<<dim3(count / 3, 3), AUX_BLOCK, 0, stream>>>(*a, (a->W + ET - 1) / ET);
+  } else {
+    const int strips_x = (a->W + EW - 1) / EW;
+    count = strips_x * ((a->H + rows - 1) / rows) * 3;
+    eval_kernel<<<8 * ((count + 7) / 8), 64, 0, stream>>>(*a, strips_x, count / 3, rows);
+  }
+  aux_reduce_kernel<<<1, 1024, 0, stream>>>(a->partials, count, 1, 1.f, a->loss_accum, 4);
   return (int)hipGetLastError();
 }

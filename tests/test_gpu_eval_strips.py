@@ -1,5 +1,6 @@
-"""The eval metrics (eval_kernel in b2ctrain_amd/csrc/kernels/aux_loss.hip) at sizes around one 54-column strip and the
-ends of its strip heights, with and without the target's alpha as weight, against the CPU oracle. Bound: the sums
+"""The eval metrics (b2ctrain_amd/csrc/kernels/aux_loss.hip) against the CPU oracle, with and without the target's alpha as
+weight: the tile kernel of small and of narrow images at sizes around one 16x16 tile, and the strip kernel at strip heights
+of 23, 34, 67 and 122 rows with ragged last strips in either direction. Bound: the sums
 are of at most W H terms in [-1, 1]; a term's fp32 blurs differ from the oracle's by roundings (1e-5 of it), its
 squared error by none that matters."""
 import numpy as np
@@ -13,7 +14,9 @@ from tests.gpu_harness import emit
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("W,H", [(1, 1), (7, 97), (54, 23), (55, 24), (53, 46), (109, 131), (640, 363)])
+@pytest.mark.parametrize("W,H", [(1, 1), (7, 97), (54, 23), (55, 24), (53, 46), (109, 131), (640, 363),
+                                 (16, 16), (17, 15), (16, 30000),
+                                 (600, 610), (163, 3001), (54, 9001), (1600, 900), (2001, 1201), (3800, 2155)])
 @pytest.mark.parametrize("mask_weighted", [False, True])
 def test_eval_strips(W, H, mask_weighted):
     sc = S.config1()
