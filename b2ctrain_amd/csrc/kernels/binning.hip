@@ -30,8 +30,12 @@ constexpr int SORT_THREADS = 256;
 // (6M, 1M splats), 142 -> 132 us (0.9M, 100k splats). 1024 threads over 16384-key tiles: 3233 and 1550 us.
 constexpr int SCATTER_THREADS = 2 * SORT_THREADS;
 constexpr int KPT_SMALL = 8;   // 2048-key tiles
-constexpr uint32_t BIG_SORT_MIN = 1u << 22;
-constexpr int KPT_BIG = 16;    // 4096-key tiles
+constexpr int KPT_BIG = 16;    // 4096-key tiles, from BIG_SORT_MIN keys
+// Sorts of 32 bits with one value, and of 17 bits with two, 2048- against 4096-key tiles: 77.7 and 85.3, 57.3 and 49.3 us
+// at 1.5M keys; 95.4 and 96.8, 70.4 and 54.1 us at 2.5M; 103.4 and 95.2, 79.3 and 55.1 us at 3M; 123.8 and 107.5, 97.0 and
+// 69.5 us at 4M. (Widths that are no bit or two over a multiple of 8 cross there too: 16 bits 41.6 and 46.1, 52.3 and 49.8,
+// 57.7 and 50.8 us.)
+constexpr uint32_t BIG_SORT_MIN = 5u << 19;
 constexpr int KPT_HUGE = 32;   // 8192-key tiles, from HUGE_SORT_MIN keys
 constexpr uint32_t HUGE_SORT_MIN = 1u << 25;
 // Up to FUSE_TILES tiles (131072 keys, their number known to the host) the histograms stay raw and by tile, and each

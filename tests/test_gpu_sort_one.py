@@ -1,5 +1,5 @@
-"""The small sorts of csrc/kernels/binning.hip: one workgroup (up to 4096 keys) at the edges of its waves and rounds, and up to
-64 tiles without a digit scan, against
+"""The small sorts of csrc/kernels/binning.hip: one workgroup (up to 4096 keys) at the edges of its waves and rounds, up to
+64 tiles without a digit scan, and the change from 2048- to 4096-key tiles, against
 numpy's stable argsort; the same keys with a second value array take the general passes and must agree too."""
 import numpy as np
 import pytest
@@ -37,6 +37,17 @@ def test_scatter_sums_the_tiles_before_it(n, begin, end, two):
     rng = np.random.default_rng(n + end)
     k, v, v2 = (rng.integers(0, 2 ** 32, n, dtype=np.uint64).astype(np.uint32) for _ in range(3))
     k[rng.random(n) < 0.3] = 0xFFFFFFFF
+    got, want = _sort(k, v, v2 if two else None, begin, end), _expect(k, v, v2 if two else None, begin, end)
+    for g, w in zip(got, want):
+        assert (g is None and w is None) or np.array_equal(g, w)
+
+
+@pytest.mark.parametrize("n", [(5 << 19) - 1, 5 << 19, (5 << 19) + 4097])
+@pytest.mark.parametrize("begin,end,two", [(0, 32, False), (0, 17, True)])
+def test_both_sides_of_the_large_tiles(n, begin, end, two):
+    """From 5 2^19 keys on a tile holds 4096 instead of 2048 of them, and 17 bits are two passes instead of three."""
+    rng = np.random.default_rng(n + end)
+    k, v, v2 = (rng.integers(0, 2 ** 32, n, dtype=np.uint64).astype(np.uint32) for _ in range(3))
     got, want = _sort(k, v, v2 if two else None, begin, end), _expect(k, v, v2 if two else None, begin, end)
     for g, w in zip(got, want):
         assert (g is None and w is None) or np.array_equal(g, w)
