@@ -165,7 +165,7 @@ __global__ void __launch_bounds__(64) evidence_kernel(b2c_evidence_args a) {
         const bool valid = (j < last_rel) & (sigma <= g1.z);
         const float alpha = valid ? fminf(ALPHA_MAX, fragment_alpha(sigma, g1.y)) : 0.f;
         const float vis = alpha * T;
-        T = T * (1.f - alpha);
+        T = __builtin_fmaf(-alpha, T, T);  // as the forward rounds it
         s_vis[j * VSTRIDE + lane] = vis;
       }
       __syncthreads();
