@@ -1,11 +1,13 @@
 """The raster's quadrant test by nearest lines (quadrant_reach in b2ctrain_amd/csrc/kernels/raster_common.h), restated
 in float32 numpy with the hardware reciprocal and square root anywhere within 1 ulp, over the splats of
-test_quadrant_cull.py: a quadrant with a pixel that passes the cutoff is kept, pixels exactly on the cutoff
-included, and no more is kept than by the minimum over each quadrant's edges but for the margins."""
+quadrant_util.py: a quadrant with a pixel that passes the cutoff is kept, pixels exactly on the cutoff
+included, and no more is kept than by the minimum over each quadrant's edges but for the margins. The GPU parity tests
+check the device code itself (a wrongly culled fragment changes the rendered colour by at least alpha = 1/255 of
+its weight)."""
 import numpy as np
 import pytest
 
-from test_quadrant_cull import _splats, pixel_truth, quadrant_mask_all_edges, sigma_at
+from tests.quadrant_util import _splats, pixel_truth, quadrant_mask_all_edges, sigma_at
 
 f32 = np.float32
 
@@ -45,21 +47,35 @@ def quadrant_reach(mx, my, ah, b, ch, power, x0, y0, rng):
         return sum(np.where(m, np.uint32(1 << k), np.uint32(0)) for k, m in enumerate(q)).astype(np.uint32)
 
 
-@pytest.mark.parametrize("spread,ratio", [(3.0, 2.0), (10.0, 5.0), (1.0, 9.2), (5.0, 11.5), (40.0, 9.2), (1000.0, 11.5)])
+@pytest.mark.parametrize("spread,ratio", [(3.0, 2.0), (10.0, 5.0), (1.0, 9.2), (5.0, 11.5), (30.0, 9.2), (40.0, 9.2),
+                                          (100.0, 11.5), (1000.0, 11.5)])
 @pytest.mark.parametrize("on_cutoff", [False, True])
 def test_quadrant_reach_is_conservative(spread, ratio, on_cutoff):
     rng = np.random.default_rng(int(spread) + 100 * on_cutoff)
     mx, my, c00, c01, c11, power, x0, y0 = _splats(rng, 200_000, spread, ratio)
-    if on_cutoff:
-        i, j = rng.integers(0, 8, mx.size).astype(f32), rng.integers(0, 8, mx.size).astype(f32)
-        power = np.maximum(sigma_at(mx, my, c00, c01, c11, x0, y0, i, j), f32(0)).astype(f32)
+    if on_cutoff:  # one pixel of each splat passes with sigma == power (one rounded below 0, against power 0)
+        i, j = rng.integers(0, 8, mx.size), rng.integers(0, 8, mx.size)
+        sig = sigma_at(mx, my, c00, c01, c11, x0, y0, i.astype(f32), j.astype(f32))
+        power = np.maximum(sig, f32(0)).astype(f32)
     ah, ch = f32(0.5) * c00, f32(0.5) * c11
     got = quadrant_reach(mx, my, ah, c01, ch, power, x0, y0, rng)
     truth = pixel_truth(mx, my, c00, c01, c11, power, x0, y0)
-    assert not (truth & ~got).any()
+    missed = truth & ~got
+    assert not missed.any(), f"culled a reachable quadrant: {np.flatnonzero(missed)[:5]}"
+    if on_cutoff:
+        on = sig <= power
+        assert ((truth & (np.uint32(1) << (2 * (j // 4) + i // 4).astype(np.uint32))) != 0)[on].all() and on.any()
+        return
     old = quadrant_mask_all_edges(mx, my, ah, c01, ch, power, x0, y0)
-    if not on_cutoff:
-        assert np.count_nonzero(got & ~old) <= 1e-3 * mx.size
+    assert np.count_nonzero(got & ~old) <= 1e-3 * mx.size
+    if spread <= 40.0:  # both outcomes occur
+        assert np.count_nonzero(truth) > 10_000 and np.count_nonzero(~got & np.uint32(0xF)) > 10_000
+
+
+def test_quadrant_reach_centre_inside():
+    mx, my, ah, b, ch, power = (np.array([v], f32) for v in (101.0, 101.0, 0.5, 0.0, 0.5, 0.0))
+    got = quadrant_reach(mx, my, ah, b, ch, power, f32(96.5), f32(96.5), np.random.default_rng(0))
+    assert got[0] == 1 << 3  # the centre is a pixel centre of quadrant (1, 1), and nothing else is reached
 
 
 def test_quadrant_reach_degenerate():
