@@ -3,10 +3,10 @@
 // per-splat reduction of the fragment gradients over the tile's 64 pixels into v_splat[n][13].
 //
 // mode 0 (replaces raster_bwd_kernel, src/gpu/raster_bwd.cu:10-156): per-fragment gradient lanes summed over
-//   the wave by shuffles, fp32 throughout. The correctness anchor.
-// mode 1 (replaces raster_bwd_tc_kernel, src/gpu/raster_bwd_tc.cu:29-225): each lane writes four scalars
-//   per fragment (vis, v_alpha*gauss, v_sigma, refine) for a group of 16 splats; the reduction over pixels
-//   is the product basis^T (16 x 64 px) * S (64 px x 16 splats) on v_mfma_f32_16x16x32_f16, with both
+//   the wave by lane swaps and DPP adds, fp32 throughout. The correctness anchor.
+// mode 1 (replaces raster_bwd_tc_kernel, src/gpu/raster_bwd_tc.cu:29-225): each lane writes three scalars
+//   per fragment (vis, v_sigma, refine) for a group of 8 splats; the reduction over pixels is the product
+//   basis^T (16 x 64 px) * S (64 px x 16: eight columns of vis, eight of v_sigma) on v_mfma_f32_16x16x32_f16, with both
 //   operands split hi/lo in fp16 (lo scaled by 2^11 and accumulated separately in fp32), which keeps ~22
 //   bits of the fp32 inputs. The basis is [v_rgb, v_feat, 1, u, v, u^2, uv, v^2] in tile-centred pixel
 //   coordinates (u, v and their products are exact in fp16); conic and mean gradients come from the
@@ -139,7 +139,6 @@ __device__ __forceinline__ Quotients divide_both(float t, float q, float keep) {
 
 template <bool FEAT, bool HOLLOW>
 __global__ void __launch_bounds__(64) raster_bwd_fp32_kernel(b2c_raster_bwd_args a) {
-  // per-fragment sums: g0..g9, the blend weight, and with FEAT the three feature lanes; the last two unused
   // per batch splat, staged once: (mx, my, c00 / 2, c01), (D, E, F, c11 / 2), (depth, log2 opacity, -, power), proj2
   __shared__ float4 s_geo[64], s_def[64], s_shape[64], s_rgb[64];
   __shared__ float2 s_f3[FEAT ? 64 : 1];                  // proj3 (feature y, z)
@@ -188,7 +187,7 @@ __global__ void __launch_bounds__(64) raster_bwd_fp32_kernel(b2c_raster_bwd_args
       const float sigma = poly_sigma(geo.z, geo.w, def.w, def.x, def.y, def.z, pp);
       const bool in = ps.inside && lo + (uint32_t)j < ps.last && sigma <= shape.w;
       if (ballot64(in) == 0ull) continue;  // uniform
-      float val[16];
+      float val[16];  // g0..g9, the blend weight, with FEAT the three feature lanes; the last two stay zero
 #pragma unroll
       for (int k = 0; k < 16; k++) val[k] = 0.f;
       if (in) {
