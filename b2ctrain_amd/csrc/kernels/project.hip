@@ -23,8 +23,8 @@ constexpr int PROJ_BLOCK = 256;
 // splats' bbox areas are prefix-summed across the wave and test t goes to lane t mod 64 (slot_owner names its
 // splat). The 64 results of a step are one ballot, from which each splat's lane shifts its own bits into its
 // mask. A wave then costs ceil(sum of areas / 64) tile tests per lane instead of its largest bbox. (A binary search
-// for the splat, LDS atomics for the mask bits and the divisions of the tile test: 120 against 113 us on 1M splats at
-// 1080p, 968 against 845 us on a dense slab of 3M, 475 against 388 us at 4K with large splats.)
+// for the splat, LDS atomics for the mask bits and the divisions of the tile test: 111 against 107 us on 1M splats at
+// 1080p, 933 against 794 us on a dense slab of 3M, 517 against 429 us at 4K with large splats.)
 struct WaveRec {
   float mx, my, c00, c01, c11, power;
   TileTest by;
